@@ -74,8 +74,9 @@ def draw(rng):
                     n=_size(rng, 16, 4096), k=_size(rng, 16, 4096), ta=rng.random() < 0.5, tb=rng.random() < 0.5,
                     beta=beta)  # fmt: skip
     if op == "half":
-        nbasis = _size(rng, 96, 400)
-        return dict(op=op, nbasis=nbasis, nocc=max(4, nbasis // rng.choice([4, 6, 8, 10])), naux=3 * nbasis - rng.choice([0, 1, 2, 8]))
+        nbasis = _size(rng, 96, 384)
+        nocc = max(4, nbasis // rng.choice([5, 6, 8, 10]))
+        return dict(op=op, nbasis=nbasis, nocc=nocc, naux=3 * nbasis - rng.choice([0, 1, 2, 8]))
     if op == "syrk":
         return dict(op=op, dtype=rng.choice(["f32", "f32", "bf16"]), n=_size(rng, 64, 4096), k=_size(rng, 64, 8192),
                     trans=rng.random() < 0.5, uplo=rng.choice(["lower", "upper"]), beta=beta)  # fmt: skip
