@@ -293,6 +293,17 @@ int trnblas_hip_mp2_energy(int64_t ic, int64_t nocc, int64_t nvir, const float* 
                            const float* eps_vir, double* out_pairs, void* stream);
 
 /*
+ * The same energies in nsplit >= 1 partial sums per pair (out: device
+ * double[ic*nocc][nsplit]; a pair's energy is the sum of its nsplit values,
+ * zeros past its tile pairs), one workgroup each: for blocks of few pairs,
+ * which would leave most of the chip idle with one workgroup per pair.
+ */
+int trnblas_hip_mp2_energy_split(int64_t ic, int64_t nocc, int64_t nvir, const float* T_flat,
+                                 int64_t ldt, const float* eps_occ_chunk,
+                                 const float* eps_occ_full, const float* eps_vir, int64_t nsplit,
+                                 double* out, void* stream);
+
+/*
  * Ozaki split of a finite fp64 matrix into `slices` int8 digits (per row or
  * per column), as trnblas/ozaki.py:123-219 `split` (digit_0 = rint(x 2^(6-e)),
  * digit_s = rint(2^7 * remainder), |digit| <= 64, e = frexp exponent of the

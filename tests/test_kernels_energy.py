@@ -160,6 +160,29 @@ def test_mp2_energy_kernel(dev):
     assert abs(float(got.sum()) - float(want)) <= 1e-9 * abs(float(want))
 
 
+@pytest.mark.parametrize("ic,nocc,nvir", [(1, 1, 1), (1, 2, 3), (2, 3, 63), (1, 3, 64), (2, 2, 65),
+                                          (1, 1, 131), (3, 700, 7), (1, 2, 200)])
+def test_mp2_energy_partials_edges(dev, ic, nocc, nvir):
+    # Tile edges (64), one pair split over workgroups, more pairs than
+    # workgroups, a row stride past the row; per pair against fp64, whose own
+    # rounding (1e-12) is the only difference: both sum fp64 terms.
+    from trnblas_amd.hip import kernels
+
+    g = torch.Generator().manual_seed(nvir)
+    wide = torch.randn(ic * nvir, nocc * nvir + 3, generator=g)
+    eo = -1.5 + torch.rand(nocc, generator=g)
+    ev = 0.1 + torch.rand(nvir, generator=g)
+    T = wide[:, 1 : 1 + nocc * nvir]
+    e = kernels.mp2_energy_partials(wide.to(dev)[:, 1 : 1 + nocc * nvir], eo[:ic].to(dev), eo.to(dev), ev.to(dev))
+    assert e.shape[0] == ic * nocc
+    T4 = T.double().reshape(ic, nvir, nocc, nvir).permute(0, 2, 1, 3)
+    vv = ev.double()[:, None] + ev.double()[None, :]
+    d = eo[:ic].double()[:, None, None, None] + eo.double()[None, :, None, None] - vv
+    want = (T4 * (2.0 * T4 - T4.mT) / d).sum((2, 3)).flatten()
+    mag = (T4.abs() * (2.0 * T4.abs() + T4.mT.abs()) / d.abs()).sum((2, 3)).flatten()
+    assert ((e.sum(1).cpu() - want).abs() <= 1e-12 * mag).all()
+
+
 @pytest.mark.parametrize("seed", [0])
 @pytest.mark.parametrize("math", MATHS)
 def test_pair_energy_config3_shape_subset(dev, seed, math):

@@ -93,6 +93,10 @@ SIGNATURES = {
         _c_int,
         [_c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr],
     ),
+    "trnblas_hip_mp2_energy_split": (
+        _c_int,
+        [_c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr],
+    ),
     "trnblas_hip_ozaki_split": (
         _c_int,
         [_c_int, _c_i64, _c_i64, _c_ptr, _c_i64, _c_int, _c_ptr, _c_i64, _c_i64, _c_ptr]

@@ -1217,7 +1217,7 @@ def nki_mp2_energy(T_flat, eps_occ_chunk, eps_occ_full, eps_vir):
 
     dev = _gpu_device(T_flat, eps_occ_chunk, eps_occ_full, eps_vir)
     try:
-        e = kernels.mp2_energy_pairs(t.to(dev), eoc.to(dev), eof.to(dev), ev.to(dev)).sum()
+        e = kernels.mp2_energy_partials(t.to(dev), eoc.to(dev), eof.to(dev), ev.to(dev)).sum()
         return _as_result_dtype(e, dt).to(T_flat.device)
     except Exception as exc:  # noqa: BLE001
         _kernel_failed(exc)

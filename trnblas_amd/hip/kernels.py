@@ -488,25 +488,41 @@ def pair_energies(
     return out
 
 
-def mp2_energy_pairs(T_flat, eps_occ_chunk, eps_occ_full, eps_vir) -> torch.Tensor:
-    """Per-pair MP2 energies (ic * nocc,) float64 of a precomputed T_flat
-    (ic * nvir, nocc * nvir) fp32 (row stride >= nocc * nvir)."""
+# Workgroups of an mp2_energy launch: eight per CU (four waves each, which
+# hide the loads of each other's tile pairs); blocks of fewer pairs are split.
+_MP2_GROUPS = 2048
+_MP2_TILE = 64
+
+
+def mp2_energy_partials(T_flat, eps_occ_chunk, eps_occ_full, eps_vir) -> torch.Tensor:
+    """MP2 energies (ic * nocc, nsplit) float64 of a precomputed T_flat
+    (ic * nvir, nocc * nvir) fp32 (row stride >= nocc * nvir): each pair's
+    energy in nsplit partial sums (the split depends on the sizes only)."""
     dev = _require_device(T_flat, eps_occ_chunk, eps_occ_full, eps_vir)
     if T_flat.dtype != torch.float32:
         raise TypeError("mp2_energy kernel takes float32 T_flat")
     if T_flat.stride(1) != 1:
         T_flat = T_flat.contiguous()
     ic, nocc, nvir = eps_occ_chunk.numel(), eps_occ_full.numel(), eps_vir.numel()
-    out = torch.empty(ic * nocc, dtype=torch.float64, device=dev)
+    nb = -(-nvir // _MP2_TILE)
+    nsplit = max(1, min(nb * (nb + 1) // 2, -(-_MP2_GROUPS // max(1, ic * nocc))))
+    out = torch.empty((ic * nocc, nsplit), dtype=torch.float64, device=dev)
     f32 = torch.float32
     eoc = eps_occ_chunk.to(f32).contiguous()
     eof = eps_occ_full.to(f32).contiguous()
     ev = eps_vir.to(f32).contiguous()
     call(
-        "trnblas_hip_mp2_energy", ic, nocc, nvir, ptr(T_flat), T_flat.stride(0) if ic else 1,
-        ptr(eoc), ptr(eof), ptr(ev), ptr(out), stream_of(dev),
+        "trnblas_hip_mp2_energy_split", ic, nocc, nvir, ptr(T_flat), T_flat.stride(0) if ic else 1,
+        ptr(eoc), ptr(eof), ptr(ev), nsplit, ptr(out), stream_of(dev),
     )  # fmt: skip
     return out
+
+
+def mp2_energy_pairs(T_flat, eps_occ_chunk, eps_occ_full, eps_vir) -> torch.Tensor:
+    """Per-pair MP2 energies (ic * nocc,) float64 (mp2_energy_partials summed
+    per pair)."""
+    e = mp2_energy_partials(T_flat, eps_occ_chunk, eps_occ_full, eps_vir)
+    return e[:, 0] if e.shape[1] == 1 else e.sum(1)
 
 
 # ── metric stage ─────────────────────────────────────────────────────────────
