@@ -597,3 +597,36 @@ def test_pack_k_kernel(dev, dtype, R, K, kp, layout):
     assert P.shape == ref.shape and P.is_contiguous()
     assert torch.equal(P.view(torch.int16 if dtype != torch.float32 else torch.int32),
                        ref.view(torch.int16 if dtype != torch.float32 else torch.int32))
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize(
+    "M,N,K,batch",
+    # each kernel of the fp32 cost model (32 x 32 tiles with K split over 4 and
+    # 8 waves, 32 x 64, 64 x 64 whole and split along K, 48 x 128, 64 x 128), at
+    # sizes one off its tile and k steps, and single rows, columns and k
+    [(1, 1, 1, 1), (3, 1, 2, 1), (33, 31, 17, 1), (97, 65, 127, 3), (129, 130, 33, 5), (257, 255, 1029, 1),
+     (65, 63, 5001, 1), (511, 513, 700, 1), (700, 1027, 513, 1), (45, 30001, 65, 1), (48, 60001, 65, 1),
+     (1, 4099, 31, 1), (4099, 1, 33, 1), (1151, 1601, 129, 1), (1025, 2050, 70, 2)],
+)
+def test_sgemm_any_alignment(dev, M, N, K, batch, ta, tb):
+    # fp32 GEMM in place on ragged operands whose neighbours hold NaN: a group
+    # loaded past a row's end must not reach the result. Against fp64 at the
+    # fp32 gate (1e-6 |A||B| + |C|).
+    from trnblas_amd.hip import kernels
+
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 7 * K)
+
+    def operand(r, c):  # a (batch, r, c) view inside a NaN-filled buffer, odd leading dimension
+        full = torch.full((batch, r, c + 3), float("nan"), device=dev)
+        full[:, :, :c] = torch.randn(batch, r, c, generator=g, device=dev)
+        return full[:, :, :c]
+
+    A = operand(K, M).mT if ta else operand(M, K)
+    B = operand(N, K).mT if tb else operand(K, N)
+    C = operand(M, N)
+    D = kernels.gemm(A[0], B[0], 1.5, -0.5, C[0])[None] if batch == 1 else kernels.gemm(A, B, 1.5, -0.5, C)
+    Ad, Bd = A.double(), B.double()
+    ref = 1.5 * (Ad @ Bd) - 0.5 * C.double()
+    den = 1.5 * (Ad.abs() @ Bd.abs()) + 0.5 * C.double().abs()
+    assert ((D.double() - ref).abs() / den).max().item() <= 1e-6

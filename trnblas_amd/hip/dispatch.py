@@ -678,9 +678,9 @@ _kernels = None  # the kernels module, once imported
 def gemm_fast(alpha, A, B, beta, C, transA, transB):
     """level3.gemm's common case without the general routing: 2-D fp32
     operands on one GPU, no gradient, the native GEMM policy auto or hip,
-    each operand row-major or a transposed row-major view that the kernel
-    reads in place (16-byte aligned, leading dimension and contiguous extent
-    multiples of 4), C absent or of the result's shape with unit column
+    each operand row-major or a transposed row-major view that the kernels
+    read in place (16-byte aligned; ragged leading dimensions and extents below
+    the size from which the general path packs them), C absent or of the result's shape with unit column
     stride. Returns alpha op(A) op(B) + beta C, or None (the general path
     then decides, as for every other call; also on a library error, which
     the general path reports). The route is the one `_gemm_route` gives
@@ -735,8 +735,8 @@ def gemm_fast(alpha, A, B, beta, C, transA, transB):
     else:
         return None
     pa, pb = A.data_ptr(), B.data_ptr()
-    if (pa | pb) & 15 or (lda | ldb | aext | bext) & 3:
-        return None
+    if (pa | pb) & 15 or ((lda | ldb | aext | bext) & 3 and M * N * K >= kern._pack_min_macs(4)):
+        return None  # (the latter are packed first)
     c, ldc, cb = 0, N, 0.0
     if C is not None and beta != 0.0:
         if (

@@ -94,18 +94,22 @@ def _batched_layout(X: torch.Tensor):
 # The GEMM / SYRK launcher moves operand panels by LDS DMA only when every
 # 16-byte group of an operand lies wholly inside or outside the matrix: a
 # 16-byte aligned base, and a leading dimension, batch stride and contiguous
-# extent that are multiples of 16 bytes. Other operands run on the
-# register-staged kernel: on the MI355X 74 TFLOP/s fp32 at 4095^3 and 8191^3
-# (the DMA kernel after packing: 126 and 132) and 81 TFLOP/s bf16 at 4095^3
-# (737 after packing). From PACK_MIN_MACS multiply-adds per launch on (by
-# element size), such operands are first copied by trnblas_hip_pack_k into
-# fresh K-contiguous buffers whose rows are padded with zeros to a multiple
-# of 16 bytes (zero products add nothing to any sum; the reference pads its
-# kernel operands the same way, nki/dispatch.py:2344-2368) and the product
-# takes the DMA kernel. Below it the two pack launches cost more than they
-# save (fp32 767^3: 40 us in place, 45 us packed; 1023^3: 52 and 52;
-# 1535^3: 126 and 99; bf16 511^3: 29 and 32; 767^3: 38 and 34).
+# extent that are multiples of 16 bytes. Other operands run on
+# register-staged kernels: fp32 GEMM at any alignment on sgemm.hip's (72-125
+# TFLOP/s from 1535^3 up), the rest at 74 TFLOP/s fp32 SYRK and 81 TFLOP/s
+# bf16 at 4095^3 (737 after packing). From PACK_MIN_MACS multiply-adds per
+# launch on, such operands are first copied by trnblas_hip_pack_k into fresh
+# K-contiguous buffers whose rows are padded with zeros to a multiple of 16
+# bytes (zero products add nothing to any sum; the reference pads its kernel
+# operands the same way, nki/dispatch.py:2344-2368) and the product takes the
+# DMA kernel. Below it the pack launches cost more than they save (bf16 511^3
+# 29 us in place, 32 packed; 767^3 38 and 34). An fp32 GEMM, whose kernels read
+# any alignment, packs from F32_GEMM_PACK_FACTOR times that size: over random
+# unaligned shapes packing is 1.6x slower than in place at 2^30 multiply-adds,
+# 1.26x at 2^33, 1.12x at 2^36, where cubes are even (4095^3 1100 us packed,
+# 1186 in place).
 PACK_MIN_MACS = {4: 1 << 30, 2: 1 << 28}
+F32_GEMM_PACK_FACTOR = 64
 
 # TRNBLAS_GEMM_RAGGED=0 restores the reference's pad-first path
 # (nki/dispatch.py:144-151, read at import as there): every operand the DMA
@@ -116,8 +120,10 @@ _RAGGED_ENABLED: bool = os.environ.get("TRNBLAS_GEMM_RAGGED", "1").strip().lower
 )  # fmt: skip
 
 
-def _pack_min_macs(elem_size: int) -> int:
-    return PACK_MIN_MACS[elem_size] if _RAGGED_ENABLED else 0
+def _pack_min_macs(elem_size: int, syrk: bool = False) -> int:
+    if not _RAGGED_ENABLED:
+        return 0
+    return PACK_MIN_MACS[elem_size] * (F32_GEMM_PACK_FACTOR if elem_size == 4 and not syrk else 1)
 
 
 def _dma_ready(t: torch.Tensor, ld: int, stride: int, ext: int, ev: int) -> bool:
@@ -164,7 +170,7 @@ def _packed_syrk_operand(A, trans, a, t, lda, n, k):
     """SYRK's (a, t, lda, k) for op(A) (n, k): as laid out, or packed
     K-contiguous with k padded to a multiple of 16 bytes (see _packed_operands)."""
     ev = 16 // A.element_size()
-    if n * n * k < _pack_min_macs(A.element_size()) or n == 0 or k == 0 or _dma_ready(a, lda, 0, n if t else k, ev):
+    if n * n * k < _pack_min_macs(A.element_size(), True) or n == 0 or k == 0 or _dma_ready(a, lda, 0, n if t else k, ev):
         return a, t, lda, k
     kp = -(-k // ev) * ev
     return _pack_k(A.t() if trans else A, kp), False, kp, kp
