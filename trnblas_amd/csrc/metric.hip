@@ -21,14 +21,19 @@
 // and the accumulator layout (lane l, register e: row 4 e + l / 16, column
 // l % 16) fall on distinct banks.
 //
-// Cholesky, per 16-wide block column p (one barrier after each phase):
-//  1. one wave factors the 16 x 16 diagonal sub-block and inverts it
-//     (diag16: column by column, the column and the multipliers' row
-//     exchanged through LDS; the inverse is built from the same row
-//     operations applied to the identity);
-//  2. the sub-blocks below it become L_ip = A_ip (L_pp^-1)^T (MFMA);
-//  3. the trailing sub-blocks lose L_ip L_kp^T (MFMA).
-// Inverse (both kernels), with the diagonal sub-blocks' inverses in place:
+// Cholesky: a serial chain of 128 columns, so everything else runs beside
+// it. Per 16-wide block column p (two barriers):
+//  A. the sub-blocks below the diagonal one become L_ip = A_ip (L_pp^-1)^T,
+//     one wave each (MFMA);
+//  B. wave 0 updates sub-block (p + 1, p + 1) with L_{p+1,p} and factors and
+//     inverts it (chol16: no memory access on its column chain); the other
+//     waves meanwhile apply the rest of the trailing update and form block
+//     row p of the inverse, Y_pj = -Y_pp sum_k L_pk Y_kj.
+// L and Y go to memory from the registers they are formed in. 27 us a
+// block under the tracer (46 us with the diagonal sub-block's columns exchanged through LDS,
+// its factorisation and the trailing update one after the other, and the
+// inverse by recursive doubling after all of them).
+// trinv128: the 8 diagonal sub-blocks inverted at once (inv16), then
 // recursive doubling over halves of 16, 32 and 64,
 // Y21 = -Y22 (L21 Y11), in place over L21, through an LDS scratch for the
 // intermediate product.
@@ -118,39 +123,114 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// v from lane SRC of the lane's 16-lane row (DPP row_newbcast).
+// v from lane SRC of the lane's 16-lane row (DPP row_newbcast: every lane has
+// a source, so the destination's old value does not matter).
 template <int SRC>
 __device__ __forceinline__ double row_bcast(double v) {
   const long long b = __builtin_bit_cast(long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b, 0x150 + SRC, 0xf, 0xf, false);
-  const unsigned hi =
-      (unsigned)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + SRC, 0xf, 0xf, false);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)b, 0x150 + SRC, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(b >> 32), 0x150 + SRC, 0xf, 0xf, true);
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// One wave on a 16 x 16 diagonal sub-block `blk` (lower part read).
-// CHOL: blk becomes L (blk = L L^T, zeros above) and inv receives L^-1;
-// a non-positive (or NaN) pivot sets *bad to min(*bad, col0 + column + 1)
-// when that column is below nb. Otherwise blk is lower triangular (unit:
-// its diagonal taken as ones) and inv receives its inverse; blk is not
-// written.
-// Lane (h = l / 16, r = l % 16) holds columns 4 e + h of row r (e = 0..3)
-// of the matrix and of E, the product of the elimination steps so far
-// (unit lower; after the last column E = (unit L)^-1, and L^-1 = diag(1 /
-// l_rr) E). Per column c: the pivot by readlane; every lane publishes its
-// (scaled) element of column 4 (c / 4) + h through LDS, of which the
-// column-c ones are read back (L[r][c] and L[s][c] for the lane's
-// columns); row c of E comes from lane c of the lane's own 16-lane row
-// (DPP). Updates are unconditional where the arithmetic leaves the final
-// values unchanged (zero multipliers, zero entries of E), so the loop has
-// no branches; the strict upper part of the matrix collects garbage that
-// is never read and is written out as zeros. ex: 80 doubles of this
+// One wave on a 16 x 16 diagonal sub-block `blk` (lower part read, SPD):
+// blk becomes L^-1 (blk = L L^T); in register e of lane (h = l / 16,
+// r = l % 16), l receives L[r][4 e + h] and y L^-1[4 e + h][r]. Returns 0, or
+// column + 1 of the first pivot that is not positive (or NaN) among the
+// leading nb columns.
+//
+// Elimination without square roots, U D U^T, four columns at a time: every
+// 16-lane row h of the wave holds the four columns of row r (p) and
+// eliminates them by itself, the pivots and multipliers' rows coming from
+// other lanes of the row by DPP, with no memory access. The steps act on a
+// 4-column identity as well (column h of it on row h: w), and then one MFMA
+// applies them to the rest of the matrix (S -= M P^T, rank 4) and one to the
+// inverse (E = W E_4 + the rows of E outside the four). S is kept whole, so
+// that by its symmetry an accumulator register t (row 4 t + h, column r) is
+// column 4 t + h of row r, the next four columns. Then L = U D^1/2 and L^-1 =
+// D^-1/2 E, the 16 inverse roots at once. A lone wave issues an instruction
+// every 7 cycles or so, which bounds this: column by column on the whole block
+// the elimination took 7400 cycles, this way about 4100. ex: 64 doubles of LDS.
+__device__ __forceinline__ int chol16(double* blk, double* ex, int lane, int nb, f64x4& l, f64x4& y) {
+  // (an opaque copy of the lane index: otherwise the per-column lane masks
+  // are computed once, outside the caller's loop, and spill)
+  asm volatile("" : "+v"(lane));
+  const int r = lane & 15, h = lane >> 4;
+  f64x4 S, E;
+  double p[4], u[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = blk[min(r, e) * kSP + max(r, e)];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int s = 4 * e + h;
+    S[e] = blk[min(r, s) * kSP + max(r, s)];
+    E[e] = s == r ? 1.0 : 0.0;
+  }
+  double mine = 1.0;  // lanes h = r % 4: the pivot of column r
+  static_for<4>([&](auto tI) {
+    constexpr int t = decltype(tI)::value;
+    double mh = 0.0, uh = 0.0;        // multiplier and value of column 4 t + h
+    double w = r == 4 * t + h ? 1.0 : 0.0;  // W[r][h]
+    static_for<4>([&](auto kI) {
+      constexpr int k = decltype(kI)::value, c = 4 * t + k;
+      const double d = row_bcast<c>(p[k]);
+      // 1 / d: the hardware estimate x and one step x (1 + e + e^2), e = 1 - d x
+      double rd = __builtin_amdgcn_rcp(d);
+      const double er = fma(-d, rd, 1.0);
+      rd = fma(rd, fma(er, er, er), rd);
+      const double m = r > c ? p[k] * rd : 0.0;
+      static_for<3 - k>([&](auto sI) {
+        constexpr int s = k + 1 + decltype(sI)::value;
+        p[s] = fma(-m, row_bcast<4 * t + s>(p[k]), p[s]);
+      });
+      w = fma(-m, row_bcast<c>(w), w);
+      mh = h == k ? m : mh;
+      uh = h == k ? p[k] : uh;
+    });
+    u[t] = uh;
+    mine = r == 4 * t + h ? uh : mine;
+    if constexpr (t < 3) {
+      S = __builtin_amdgcn_mfma_f64_16x16x4f64(-mh, uh, S, 0, 0, 0);
+      ex[lane] = S[t + 1];
+    }
+    const double e4 = E[t];
+    E[t] = 0.0;
+    E = __builtin_amdgcn_mfma_f64_16x16x4f64(w, e4, E, 0, 0, 0);
+    if constexpr (t < 3) {
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int k = 0; k < 4; ++k) p[k] = ex[16 * k + r];
+      __builtin_amdgcn_wave_barrier();
+    }
+  });
+  // the lane that holds the pivot of column r
+  const bool own = (r & 3) == h;
+  const unsigned long long b = __ballot(own && !(mine > 0.0) && r < nb);
+  const unsigned cols = (unsigned)(b | b >> 16 | b >> 32 | b >> 48) & 0xffffu;
+  if (own) ex[r] = rsqrt_nr(mine);
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int s = 4 * e + h;
+    const double rs = ex[s];
+    l[e] = u[e] * rs;
+    y[e] = s >= r ? E[e] * rs : 0.0;
+    blk[r * kSP + s] = y[e];
+  }
+  return cols ? (int)__builtin_ctz(cols) + 1 : 0;
+}
+
+// One wave on a 16 x 16 lower triangular sub-block `blk` (unit: its diagonal
+// taken as ones), in place: blk becomes its inverse. Lane (h = l / 16,
+// r = l % 16) holds columns 4 e + h of row r (e = 0..3) of the matrix and of
+// E, the product of the elimination steps (the inverse is diag(1 / t_rr) E).
+// Per column c every lane publishes its element of column 4 (c / 4) + h
+// through LDS, of which the column-c ones are read back; row c of E comes
+// from lane c of the lane's own 16-lane row (DPP). ex: 80 doubles of this
 // wave's LDS.
-template <bool CHOL>
-__device__ __forceinline__ void diag16(double* blk, double* inv, double* ex, int lane, bool unit,
-                                       int* bad, int col0, int nb) {
+__device__ __forceinline__ void inv16(double* blk, double* ex, int lane, bool unit) {
   double* colb = ex;        // colb[16 h + r]: lane (h, r)'s published value
-  double* rinvb = ex + 64;  // 1 / l_cc
+  double* rinvb = ex + 64;  // 1 / t_cc
   // (an opaque copy of the lane index: otherwise the per-column lane masks
   // are computed once, outside the caller's loop, and spill)
   int ln = lane;
@@ -161,45 +241,29 @@ __device__ __forceinline__ void diag16(double* blk, double* inv, double* ex, int
   for (int e = 0; e < 4; ++e) {
     const int s = 4 * e + h;
     a[e] = s <= r ? blk[s * kSP + r] : 0.0;
-    if (!CHOL && unit && s == r) a[e] = 1.0;
+    if (unit && s == r) a[e] = 1.0;
     E[e] = s == r ? 1.0 : 0.0;
   }
   static_for<16>([&](auto cI) {
     constexpr int c = decltype(cI)::value, ch = c & 3, ce = c >> 2;
     const double d = readlane_f64(a[ce], c + 16 * ch);  // the pivot
-    const double rinv = CHOL ? rsqrt_nr(d) : (unit ? 1.0 : rcp_nr(d));
-    colb[16 * h + r] = CHOL ? a[ce] * rinv : a[ce];
+    const double rinv = unit ? 1.0 : rcp_nr(d);
+    colb[16 * h + r] = a[ce];
     rinvb[c] = rinv;
     double ev[4];  // E[c][4 e + h]
 #pragma unroll
     for (int e = 0; e < 4; ++e) ev[e] = row_bcast<c>(E[e]);
     __builtin_amdgcn_wave_barrier();
-    const double lr = colb[16 * ch + r];  // L[r][c] (CHOL) / T[r][c]
-    const double m = r > c ? lr * rinv : 0.0;  // the elimination multiplier of row r
-    if (CHOL) {
-      double cs[4];  // L[4 e + h][c]
-#pragma unroll
-      for (int e = ce; e < 4; ++e) cs[e] = colb[16 * ch + 4 * e + h];
-      a[ce] = h == ch ? lr : a[ce];
-#pragma unroll
-      for (int e = ce + 1; e < 4; ++e) a[e] = fma(-lr, cs[e], a[e]);
-      a[ce] = h > ch ? fma(-lr, cs[ce], a[ce]) : a[ce];
-    }
+    const double m = r > c ? colb[16 * ch + r] * rinv : 0.0;  // the multiplier of row r
 #pragma unroll
     for (int e = 0; e < 4; ++e) E[e] = fma(-m, ev[e], E[e]);
     __builtin_amdgcn_wave_barrier();
   });
   const double rr = rinvb[r];
-  if (CHOL) {  // the first NaN 1 / l_cc is the first pivot that is not positive
-    const bool isbad = ln < 16 && !(rr == rr) && col0 + ln < nb;
-    const unsigned long long msk = __ballot(isbad);
-    if (msk != 0ull && ln == 0) *bad = min(*bad, col0 + (int)__builtin_ctzll(msk) + 1);
-  }
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int s = 4 * e + h;
-    if (CHOL) blk[s * kSP + r] = s <= r ? a[e] : 0.0;
-    inv[s * kSP + r] = s <= r ? E[e] * rr : 0.0;
+    blk[s * kSP + r] = s <= r ? E[e] * rr : 0.0;
   }
 }
 
@@ -295,12 +359,11 @@ __device__ __forceinline__ void load_lower(double* G, const TT* X, int64_t ri, i
   }
 }
 
-// The lower triangle of the grid out to Z[i * zr + k * zc] for i, k < nb
-// (zeros above the diagonal when `full`, else the strict upper part
-// untouched), in the thread mapping of load_lower.
+// The lower triangle of the grid out to Z[i * zr + k * zc] for i, k < nb,
+// zeros above the diagonal, in the thread mapping of load_lower.
 template <typename TT>
 __device__ __forceinline__ void store_lower(const double* G, TT* Z, int64_t zr, int64_t zc, int nb,
-                                            bool full, int tid, bool skip_diag = false) {
+                                            int tid) {
   constexpr int PER = kCholNB * kCholNB / kThreads;
   asm volatile("" : "+v"(tid));  // (its masks and addresses computed here, not at kernel entry)
   const int k = tid & 127, i0 = tid >> 7;
@@ -315,67 +378,131 @@ __device__ __forceinline__ void store_lower(const double* G, TT* Z, int64_t zr, 
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
     const int i = i0 + 4 * u;
-    if (i < nb && k < nb && (full || k <= i) && !(skip_diag && (i >> 4) == (k >> 4)))
-      z[(int64_t)(4 * u) * zr] = (TT)v[u];
+    if (i < nb && k < nb) z[(int64_t)(4 * u) * zr] = (TT)v[u];
   }
 }
 
-// LDS: the sub-block grid (78 KB), one diagonal inverse, the block
-// inverse's scratch and diag16's exchange: 91 KB, so the workgroup shares a
-// CU with a GEMM workgroup (64 KB) of a concurrent stream instead of
-// waiting for a whole free CU.
+// LDS: the sub-block grid and a 16 x 16 scratch per wave, 96 KB, so the
+// workgroup shares a CU with a GEMM workgroup (64 KB) of a concurrent
+// stream instead of waiting for a whole free CU. zero_upper: the sub-blocks
+// of Li above its diagonal ones are cleared (else they hold zeros already).
 __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, int64_t lda,
                                                            double* Li, int64_t ldl, int32_t* info,
-                                                           int offset) {
+                                                           int offset, int zero_upper) {
+  constexpr int NW = kThreads / 64;
   __shared__ double G[kNLow * kSB];
-  __shared__ double D1[kSB];        // inverse of the current diagonal sub-block
-  __shared__ double scr[4 * kSB];   // T of the block inverse
-  __shared__ double ex[80];         // diag16's exchange
-  __shared__ int sbad;
-  const int tid = threadIdx.x, lane = tid & 63;
+  __shared__ double scr[NW][kSB];  // T of the inverse's block row; chol16's exchange
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (tid == 0) sbad = 0x7fffffff;
-  // the lower triangle, the identity past nb (diag16 reads and writes only
-  // the lower part of a diagonal sub-block)
-  load_lower(G, A, lda, 1, nb, tid);
+  // sub-block (i, k) of an accumulator to Z, rows and columns below nb
+  auto put = [&](double* Z, int64_t ld, int i, int k, const f64x4& v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * i + 4 * e + lg, col = 16 * k + li;
+      if (row < nb && col < nb) Z[(int64_t)row * ld + col] = v[e];
+    }
+  };
+  // sub-block (i, k) of A, the identity past nb
+  auto get = [&](int i, int k) __attribute__((always_inline)) {
+    f64x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * i + 4 * e + lg, col = 16 * k + li;
+      v[e] = row == col ? 1.0 : 0.0;
+      if (row < nb && col <= row) v[e] = A[(int64_t)row * lda + col];
+    }
+    return v;
+  };
+  int bad = 0;  // wave 0: the first pivot that is not positive, 1-based
+  // wave 0: chol16's l and y of step p; the others: the panel sub-block and
+  // the inverse's (with its partial sum t)
+  f64x4 l = {0.0, 0.0, 0.0, 0.0}, y = l, t = l;
+  if (wave == 0) {
+    store_acc(G, lane, get(0, 0));
+    __builtin_amdgcn_wave_barrier();
+    bad = chol16(G, scr[0], lane, nb, l, y);
+  } else {  // the other 35 sub-blocks meanwhile, five per wave
+    f64x4 v[5];
+#pragma unroll
+    for (int x = 0; x < 5; ++x) {
+      const int q = wave + 7 * x;
+      int i = 0;
+      while ((i + 1) * (i + 2) / 2 <= q) ++i;
+      v[x] = get(i, q - i * (i + 1) / 2);
+    }
+#pragma unroll
+    for (int x = 0; x < 5; ++x) store_acc(G + (wave + 7 * x) * kSB, lane, v[x]);
+    if (zero_upper) {
+      for (int x = tid - 64; x < kCholNB * kCholNB; x += kThreads - 64) {
+        const int i = x >> 7, k = x & 127;
+        if ((k >> 4) > (i >> 4) && i < nb && k < nb) Li[(int64_t)i * ldl + k] = 0.0;
+      }
+    }
+  }
   __syncthreads();
   for (int p = 0; p < kNS; ++p) {
-    double* Gpp = G + sidx(p, p) * kSB;
-    if (wave == 0) diag16<true>(Gpp, D1, ex, lane, false, &sbad, 16 * p, nb);
-    __syncthreads();
-    for (int i = p + 1 + wave; i < kNS; i += kThreads / 64) {  // panel
-      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-      mma16<true>(acc, G + sidx(i, p) * kSB, D1, 1.0, lane);
-      store_acc(G + sidx(i, p) * kSB, lane, acc);
-    }
-    __syncthreads();
-    const int nt = kNS - 1 - p, items = nt * (nt + 1) / 2;
-    if (wave == 7) {
-      // L_pp out to A (its lower part), then L_pp^-1 in its place: the
-      // trailing update below does not read the diagonal sub-block
-      for (int e = lane; e < 256; e += 64) {
-        const int r = e >> 4, c = e & 15, i = 16 * p + r, k = 16 * p + c;
-        if (c <= r && i < nb) A[(int64_t)i * lda + k] = Gpp[c * kSP + r];
+    const double* D = G + sidx(p, p) * kSB;  // L_pp^-1
+    // A. the panel (wave 0 has no row of it: it stores L_pp and its inverse)
+    const int pi = p + NW - wave;
+    if (wave == 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 16 * p + li, s = 16 * p + 4 * e + lg;
+        if (r < nb && s < nb) {
+          Li[(int64_t)s * ldl + r] = y[e];
+          if (s <= r) A[(int64_t)r * lda + s] = l[e];
+        }
       }
-      for (int e = lane; e < kSB; e += 64) Gpp[e] = D1[e];
-    }
-    for (int it = wave; it < items; it += kThreads / 64) {  // trailing update
-      int ri = 0;
-      while ((ri + 1) * (ri + 2) / 2 <= it) ++ri;
-      const int i = p + 1 + ri, k = p + 1 + (it - ri * (ri + 1) / 2);
-      f64x4 acc = load_acc(G + sidx(i, k) * kSB, lane);
-      mma16<true>(acc, G + sidx(i, p) * kSB, G + sidx(k, p) * kSB, -1.0, lane);
-      store_acc(G + sidx(i, k) * kSB, lane, acc);
+    } else if (pi < kNS) {
+      l = f64x4{0.0, 0.0, 0.0, 0.0};
+      mma16<true>(l, G + sidx(pi, p) * kSB, D, 1.0, lane);
+      store_acc(G + sidx(pi, p) * kSB, lane, l);
     }
     __syncthreads();
+    // B. wave 0 the next diagonal sub-block; the others block row p of the
+    // inverse (column j on wave j + 1), the part of row p + 1 that is known,
+    // and the rest of the trailing update
+    const bool last = p + 1 == kNS;
+    if (wave == 0 && !last) {
+      double* N = G + sidx(p + 1, p + 1) * kSB;
+      const double* X = G + sidx(p + 1, p) * kSB;
+      f64x4 acc = load_acc(N, lane);
+      mma16<true>(acc, X, X, -1.0, lane);
+      store_acc(N, lane, acc);
+      __builtin_amdgcn_wave_barrier();
+      const int b = chol16(N, scr[0], lane, nb - 16 * (p + 1), l, y);
+      if (bad == 0 && b != 0) bad = 16 * (p + 1) + b;
+    } else {
+      if (pi < kNS) put(A, lda, pi, p, l);
+      const int j = wave - 1;
+      if (wave != 0 && j < p) {
+        // t holds sum_{k < p - 1} L_pk Y_kj from the step before
+        mma16<false>(t, G + sidx(p, p - 1) * kSB, G + sidx(p - 1, j) * kSB, 1.0, lane);
+        store_acc(scr[wave], lane, t);
+        __builtin_amdgcn_wave_barrier();
+        y = f64x4{0.0, 0.0, 0.0, 0.0};
+        mma16<false>(y, D, scr[wave], -1.0, lane);
+        put(Li, ldl, p, j, y);
+        t = f64x4{0.0, 0.0, 0.0, 0.0};
+        if (!last)
+          for (int k = j; k < p; ++k)
+            mma16<false>(t, G + sidx(p + 1, k) * kSB, G + sidx(k, j) * kSB, 1.0, lane);
+      }
+      const int nt = kNS - 1 - p, items = nt * (nt + 1) / 2;
+      for (int it = NW - wave; it < items; it += NW - 1) {  // item 0 is wave 0's
+        int ri = 0;
+        while ((ri + 1) * (ri + 2) / 2 <= it) ++ri;
+        const int i = p + 1 + ri, k = p + 1 + (it - ri * (ri + 1) / 2);
+        f64x4 acc = load_acc(G + sidx(i, k) * kSB, lane);
+        mma16<true>(acc, G + sidx(i, p) * kSB, G + sidx(k, p) * kSB, -1.0, lane);
+        store_acc(G + sidx(i, k) * kSB, lane, acc);
+      }
+    }
+    __syncthreads();
+    // Y_pj over L_pj, which every wave has now read
+    if (!last && wave >= 1 && wave - 1 < p) store_acc(G + sidx(p, wave - 1) * kSB, lane, y);
   }
-  // the off-diagonal sub-blocks of L out (the diagonal ones went out per
-  // step; the diagonal sub-blocks of G now hold their inverses)
-  store_lower(G, A, lda, (int64_t)1, nb, false, tid, true);
-  __syncthreads();
-  block_inverse(G, scr, wave, lane);
-  store_lower(G, Li, ldl, (int64_t)1, nb, true, tid);
-  if (tid == 0 && sbad != 0x7fffffff && info[0] == 0) info[0] = offset + sbad;
+  if (tid == 0 && bad != 0 && info[0] == 0) info[0] = offset + bad;
 }
 
 // Inverse of diagonal block b of the n x n triangular matrix T: element
@@ -396,34 +523,37 @@ __global__ __launch_bounds__(kThreads) void trinv128_kernel(int n, int upper, in
   const int64_t ri = upper ? sc : sr, ci = upper ? sr : sc;  // strides of the lower view
   load_lower(G, T + (int64_t)k0 * (sr + sc), ri, ci, nb, tid);
   __syncthreads();
-  // the 8 diagonal sub-blocks' inverses, one wave each, in place (diag16
-  // reads the sub-block into registers before it writes the inverse)
-  diag16<false>(G + sidx(wave, wave) * kSB, G + sidx(wave, wave) * kSB, ex[wave], lane, unit != 0,
-                nullptr, 0, 0);
+  // the 8 diagonal sub-blocks' inverses, one wave each, in place
+  inv16(G + sidx(wave, wave) * kSB, ex[wave], lane, unit != 0);
   __syncthreads();
   block_inverse(G, scr, wave, lane);
   // lower: out[i][k] = Y[i][k]; upper: out[k][i] = Y[i][k]
   TT* out = Dinv + (int64_t)b * kCholNB * kCholNB;
   store_lower(G, out, upper ? (int64_t)1 : (int64_t)kCholNB, upper ? (int64_t)kCholNB : (int64_t)1,
-              kCholNB, true, tid);
+              kCholNB, tid);
 }
 
 }  // namespace trnblas
 
 using namespace trnblas;
 
-extern "C" int trnblas_hip_chol_block(int64_t nb, double* A, int64_t lda, double* Linv,
-                                      int64_t ldl, int32_t* info, int64_t offset, void* stream) {
-  clear_error();
+int trnblas::chol_block(int64_t nb, double* A, int64_t lda, double* Linv, int64_t ldl,
+                        int32_t* info, int64_t offset, bool zero_upper, hipStream_t stream) {
   TRNBLAS_CHECK_ARG(nb >= 0 && nb <= kCholNB, "chol_block: nb %lld not in [0, %d]", (long long)nb,
                     kCholNB);
   if (nb == 0) return TRNBLAS_OK;
   TRNBLAS_CHECK_ARG(A && Linv && info, "chol_block: NULL pointer");
   TRNBLAS_CHECK_ARG(lda >= nb && ldl >= nb, "chol_block: leading dimension below nb");
   TRNBLAS_CHECK_ARG(offset >= 0 && offset < (1ll << 30), "chol_block: bad offset");
-  hipLaunchKernelGGL(chol128_kernel, dim3(1), dim3(kThreads), 0, (hipStream_t)stream, (int)nb, A,
-                     lda, Linv, ldl, info, (int)offset);
+  hipLaunchKernelGGL(chol128_kernel, dim3(1), dim3(kThreads), 0, stream, (int)nb, A, lda, Linv, ldl,
+                     info, (int)offset, (int)zero_upper);
   return check_launch("chol_block");
+}
+
+extern "C" int trnblas_hip_chol_block(int64_t nb, double* A, int64_t lda, double* Linv,
+                                      int64_t ldl, int32_t* info, int64_t offset, void* stream) {
+  clear_error();
+  return chol_block(nb, A, lda, Linv, ldl, info, offset, true, (hipStream_t)stream);
 }
 
 extern "C" int trnblas_hip_tri_inv_blocks(int dtype, int64_t n, int upper, int unit, const void* T,

@@ -193,7 +193,7 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
     const int64_t k0 = b * kNB, m = n - k0 < kNB ? n - k0 : kNB;
     double* Ybb = Y + k0 * npad + k0;
     // L_bb into W (lower triangle), L_bb^-1 = Y_bb straight into Y
-    TRY(trnblas_hip_chol_block(m, W + k0 * npad + k0, npad, Ybb, npad, info, k0, main));
+    TRY(chol_block(m, W + k0 * npad + k0, npad, Ybb, npad, info, k0, false, main));
     // block row b of Y: T = L[b, :b] Y[:b, :b], Y[b, :b] = -Y_bb T, on the
     // inverse stream once `ready` (recorded after this step's GEMMs on the
     // caller's stream, or right here in the last step) follows Y_bb
