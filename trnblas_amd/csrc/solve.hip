@@ -7,17 +7,21 @@
 // and gemm.hip for fp32 trsm). Issued from Python, each launch's host cost
 // (~50 us through ctypes) exceeded its GPU time, and the GPU waited.
 //
-// metric_inv_half: right-looking blocked Cholesky with look-ahead. After the
-// panel of block b only the next block column is updated on the caller's
-// stream, so block b + 1 is factored while a second stream (per device,
-// default priority) applies the rest of the trailing update (lower
-// triangle only) with the other CUs; the caller's stream waits for it
-// before it next writes there. Y = L^-1 is built beside the factorisation
-// on a third stream: once block b is factored (its inverse Y_bb written in
-// place by the diagonal kernel), block row b of Y follows from the rows
-// above it, Y[b, :b] = -Y_bb (L[b, :b] Y[:b, :b]), two GEMMs that run
-// while the caller's stream factors the next blocks (the late steps, bound
-// by the one-workgroup diagonal kernel, leave most CUs free). Then X = Y^T.
+// metric_inv_half: right-looking blocked Cholesky in steps of 256 columns
+// (two 128-wide diagonal blocks) with look-ahead. After a step's two panels
+// only the next step's columns are updated on the caller's stream, so that
+// they are factored while a second stream (per device, default priority)
+// applies the rest of the trailing update (lower triangle only, rank 256)
+// with the other CUs; the caller's stream waits for it before it next writes
+// there. Y = L^-1 is built beside the factorisation on a third stream: the
+// rows B of a step are Y[B, :k0] = -Y_BB T_B with T_B = L[B, :k0] Y[:k0, :k0],
+// which is formed before B is factored, so that only the short product
+// follows the last diagonal block. Then X = Y^T. A hand-over between streams
+// costs some 10 us beside the 35 us that the caller's stream works per 128
+// columns: with one per 128 columns, the rows' long products after their
+// diagonal block, and W and Y cleared by passes of their own, naux 384 /
+// 1024 / 2304 / 4096 took 185 / 545 / 1117 / 2500 us against 157 / 404 / 926 /
+// 2244.
 #include <mutex>
 
 #include "common.hpp"
@@ -26,16 +30,10 @@ namespace trnblas {
 
 constexpr int kNB = 128;
 
-// The 2-D helpers walk rows with blockIdx.y and columns with blockIdx.x
-// (grid-strided both ways).
-__global__ __launch_bounds__(256) void fill_kernel(double* p, int64_t rows, int64_t cols,
-                                                   int64_t ld, double v) {
-  for (int64_t i = blockIdx.y; i < rows; i += gridDim.y)
-    for (int64_t j = blockIdx.x * 256ll + threadIdx.x; j < cols; j += (int64_t)gridDim.x * 256)
-      p[i * ld + j] = v;
-}
+constexpr int kStep = 2 * kNB;  // columns of a step of metric_inv_half
 
-// dst[i * dr + j * dc] = alpha * src[i * sr + j * sc], rows x cols
+// dst[i * dr + j * dc] = alpha * src[i * sr + j * sc], rows x cols (rows by
+// blockIdx.y and columns by blockIdx.x, grid-strided both ways)
 template <typename TS, typename TD>
 __global__ __launch_bounds__(256) void copy2d_kernel(int64_t rows, int64_t cols, const TS* src,
                                                      int64_t sr, int64_t sc, TD* dst,
@@ -45,40 +43,55 @@ __global__ __launch_bounds__(256) void copy2d_kernel(int64_t rows, int64_t cols,
       dst[i * dr + j * dc] = (TD)(alpha * (double)src[i * sr + j * sc]);
 }
 
-__global__ void set_i32_kernel(int32_t* p, int32_t v) { *p = v; }
-
 static dim3 grid2d(int64_t rows, int64_t cols) {
   const int64_t gx = (cols + 255) / 256, gy = rows;
   return dim3((unsigned)(gx < 64 ? (gx > 0 ? gx : 1) : 64), (unsigned)(gy < 4096 ? (gy > 0 ? gy : 1) : 4096));
 }
 
-// X[j][i] = Y[i][j] for i, j < n through a 64 x 64 LDS tile (both sides
-// coalesced)
+// X[j][i] = Y[i][j] for j <= i < n and zeros for j > i, through a 64 x 64 LDS
+// tile (both sides coalesced; only Y's lower tiles are read)
 __global__ __launch_bounds__(256) void transpose_kernel(int n, const double* Y, int64_t ldy,
                                                         double* X, int64_t ldx) {
   __shared__ double t[64][65];
   const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int r = ty; r < 64; r += 4) {
-    const int i = i0 + r, j = j0 + tx;
-    t[r][tx] = (i < n && j < n) ? Y[(int64_t)i * ldy + j] : 0.0;
+  if (i0 >= j0) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int i = i0 + ty + 4 * r, j = j0 + tx;
+      t[ty + 4 * r][tx] = i < n && j <= i ? Y[(int64_t)i * ldy + j] : 0.0;
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  for (int r = ty; r < 64; r += 4) {
-    const int j = j0 + r, i = i0 + tx;
-    if (i < n && j < n) X[(int64_t)j * ldx + i] = t[tx][r];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int j = j0 + ty + 4 * r, i = i0 + tx;
+    if (i < n && j < n) X[(int64_t)j * ldx + i] = i0 >= j0 ? t[tx][ty + 4 * r] : 0.0;
+  }
+}
+
+// W's lower 128 x 128 blocks = J's, zeros past n; zeros in Y's last diagonal
+// block when it is partial (its padding takes part in the products); info =
+// 0. Grid: (blocks of a row, block rows, 8 slices of 16 rows).
+__global__ __launch_bounds__(256) void metric_init_kernel(int64_t n, int64_t npad, const double* J,
+                                                          int64_t ldj, double* W, double* Y,
+                                                          int32_t* info) {
+  const int64_t bi = blockIdx.y, bj = blockIdx.x;
+  if (bj > bi) return;
+  if (bi == 0 && blockIdx.z == 0 && threadIdx.x == 0) *info = 0;
+  const bool tail = bi == bj && (bi + 1) * 128 > n;
+  const int64_t j = bj * 128 + (threadIdx.x & 127);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int64_t i = bi * 128 + blockIdx.z * 16 + (threadIdx.x >> 7) + 2 * u;
+    W[i * npad + j] = i < n && j < n ? J[i * ldj + j] : 0.0;
+    if (tail) Y[i * npad + j] = 0.0;
   }
 }
 
 static int grid_for(int64_t elems) {
   const int64_t g = (elems + 255) / 256;
   return (int)(g < 4096 ? (g > 0 ? g : 1) : 4096);
-}
-
-static int fill(double* p, int64_t rows, int64_t cols, int64_t ld, double v, hipStream_t s) {
-  if (rows <= 0 || cols <= 0) return TRNBLAS_OK;
-  hipLaunchKernelGGL(fill_kernel, grid2d(rows, cols), dim3(256), 0, s, p, rows, cols, ld, v);
-  return check_launch("fill");
 }
 
 // Per device: the side stream of the look-ahead and the two events that
@@ -116,15 +129,15 @@ static int side_init(SideStream* ss) {
   return TRNBLAS_OK;
 }
 
-static void metric_layout(int64_t n, int64_t& nblk, int64_t& npad, size_t off[4]) {
-  nblk = (n + kNB - 1) / kNB;
-  npad = nblk * kNB;
+static void metric_layout(int64_t n, int64_t& npad, size_t off[5]) {
+  npad = (n + kNB - 1) / kNB * kNB;
   const size_t sq = (size_t)npad * npad * 8;
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
   off[0] = 0;                                // W: J, updated in place
   off[1] = up(off[0] + sq);                  // L: panels of the factor
   off[2] = up(off[1] + sq);                  // Y: L^-1 (diagonal blocks from the kernel)
-  off[3] = up(off[2] + sq);                  // T: a block row's product L[b, :b] Y[:b, :b]
+  off[3] = up(off[2] + sq);                  // T: a step's rows L[B, :k0] Y[:k0, :k0]
+  off[4] = up(off[3] + (size_t)kStep * npad * 8);  // S: L_10 Y_00 of a step's blocks 0, 1
 }
 
 #define TRY(x)                        \
@@ -139,10 +152,10 @@ using namespace trnblas;
 
 extern "C" size_t trnblas_hip_metric_inv_half_workspace(int64_t n) {
   if (n <= 0) return 0;
-  int64_t nblk, npad;
-  size_t off[4];
-  metric_layout(n, nblk, npad, off);
-  return off[3] + (size_t)kNB * npad * 8;
+  int64_t npad;
+  size_t off[5];
+  metric_layout(n, npad, off);
+  return off[4] + (size_t)kNB * kNB * 8;
 }
 
 extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t ldj, double* X,
@@ -159,14 +172,15 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
   TRNBLAS_CHECK_ARG((reinterpret_cast<uintptr_t>(workspace) & 255) == 0,
                     "metric_inv_half: workspace must be 256-byte aligned");
   hipStream_t main = (hipStream_t)stream;
-  int64_t nblk, npad;
-  size_t off[4];
-  metric_layout(n, nblk, npad, off);
+  int64_t npad;
+  size_t off[5];
+  metric_layout(n, npad, off);
   char* ws = static_cast<char*>(workspace);
   double* W = reinterpret_cast<double*>(ws + off[0]);
   double* L = reinterpret_cast<double*>(ws + off[1]);
   double* Y = reinterpret_cast<double*>(ws + off[2]);
   double* T = reinterpret_cast<double*>(ws + off[3]);
+  double* S = reinterpret_cast<double*>(ws + off[4]);
   int rc = TRNBLAS_OK;
   SideStream* ss = side_stream(rc);
   if (!ss) return rc;
@@ -179,67 +193,77 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
     return hipEventRecord(e, s) == hipSuccess ? TRNBLAS_OK : TRNBLAS_E_LAUNCH;
   };
 
-  // W = J zero-padded; Y = 0 (the last block's padding stays 0); info = 0
-  TRY(fill(W, npad, npad, npad, 0.0, main));
-  hipLaunchKernelGGL((copy2d_kernel<double, double>), grid2d(n, n), dim3(256), 0, main, n, n, J,
-                     ldj, (int64_t)1, W, npad, (int64_t)1, 1.0);
-  TRY(check_launch("metric_inv_half(copy)"));
-  TRY(fill(Y, npad, npad, npad, 0.0, main));
-  hipLaunchKernelGGL(set_i32_kernel, dim3(1), dim3(1), 0, main, info, 0);
-  TRY(check_launch("metric_inv_half(info)"));
+  const unsigned nblk = (unsigned)(npad / kNB);
+  hipLaunchKernelGGL(metric_init_kernel, dim3(nblk, nblk, 8), dim3(256), 0, main, n, npad, J, ldj, W,
+                     Y, info);
+  TRY(check_launch("metric_inv_half(init)"));
+  // D = alpha A op(B) + beta D over blocks of W, L, Y (ld npad)
+  auto mm = [&](bool bt, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
+                const double* B, int64_t ldb, double beta, double* D, int64_t ldd, int lower, int tri,
+                hipStream_t s) {
+    return trnblas_hip_dgemm(0, bt, M, N, K, alpha, A, npad, 0, B, ldb, 0, beta, D, ldd, 0, D, ldd,
+                             0, 1, lower, tri, s);
+  };
+  auto chol = [&](int64_t k) {  // L_bb into W (lower triangle), L_bb^-1 = Y_bb into Y
+    return chol_block(n - k < kNB ? n - k : kNB, W + k * npad + k, npad, Y + k * npad + k, npad, info,
+                      k, true, main);
+  };
 
-  bool rest = false, inv = false;  // the side / inverse stream has work pending
-  for (int64_t b = 0; b < nblk; ++b) {
-    const int64_t k0 = b * kNB, m = n - k0 < kNB ? n - k0 : kNB;
-    double* Ybb = Y + k0 * npad + k0;
-    // L_bb into W (lower triangle), L_bb^-1 = Y_bb straight into Y
-    TRY(chol_block(m, W + k0 * npad + k0, npad, Ybb, npad, info, k0, false, main));
-    // block row b of Y: T = L[b, :b] Y[:b, :b], Y[b, :b] = -Y_bb T, on the
-    // inverse stream once `ready` (recorded after this step's GEMMs on the
-    // caller's stream, or right here in the last step) follows Y_bb
-    auto inv_row = [&]() -> int {
-      if (b == 0) return TRNBLAS_OK;
-      TRY(wait(ss->inv, ss->ready));
-      TRY(trnblas_hip_dgemm(0, 0, kNB, k0, k0, 1.0, L + k0 * npad, npad, 0, Y, npad, 0, 0.0,
-                            nullptr, npad, 0, T, npad, 0, 1, 0, TRNBLAS_TRI_B_LOWER, ss->inv));
-      TRY(trnblas_hip_dgemm(0, 0, kNB, k0, kNB, -1.0, Ybb, npad, 0, T, npad, 0, 0.0, nullptr,
-                            npad, 0, Y + k0 * npad, npad, 0, 1, 0, TRNBLAS_TRI_A_LOWER, ss->inv));
-      inv = true;
-      return TRNBLAS_OK;
-    };
-    if (k0 + kNB >= npad) {
-      if (b > 0) TRY(record(ss->ready, main));
-      TRY(inv_row());
-      break;
+  // up to two steps there is no trailing update, and the hand-overs to the
+  // inverse stream cost what it would overlap
+  hipStream_t inv = npad <= 2 * kStep ? main : ss->inv;
+  bool rest = false;  // the side stream has a trailing update pending
+  for (int64_t k0 = 0; k0 < npad; k0 += kStep) {
+    const int64_t k1 = k0 + kNB;
+    const int64_t k2 = k1 < npad ? k1 + kNB : k1;  // the step's columns k0 .. k2
+    const int64_t k3 = k2 + kStep < npad ? k2 + kStep : npad;  // the next step's end
+    double* Y00 = Y + k0 * npad + k0;
+    double* Y11 = Y + k1 * npad + k1;
+    TRY(chol(k0));
+    if (k2 > k1) {
+      const int64_t rows = npad - k1;
+      double* P = L + k1 * npad + k0;  // the panel of block 0: W[k1:, k0:k1] Y00^T
+      TRY(mm(true, rows, kNB, kNB, 1.0, W + k1 * npad + k0, Y00, npad, 0.0, P, npad, 0, 0, main));
+      TRY(mm(true, rows, kNB, kNB, -1.0, P, P, npad, 1.0, W + k1 * npad + k1, npad, 0, 0, main));
+      TRY(chol(k1));
+      if (k2 < npad)
+        TRY(mm(true, npad - k2, kNB, kNB, 1.0, W + k2 * npad + k1, Y11, npad, 0.0,
+               L + k2 * npad + k1, npad, 0, 0, main));
     }
-    const int64_t k1 = k0 + kNB, k2 = k1 + kNB, rows = npad - k1;
-    // the panel of L: L[k1:, k0:k1] = W[k1:, k0:k1] Y_bb^T
-    TRY(trnblas_hip_dgemm(0, 1, rows, kNB, kNB, 1.0, W + k1 * npad + k0, npad, 0, Ybb, npad, 0,
-                          0.0, nullptr, npad, 0, L + k1 * npad + k0, npad, 0, 1, 0, 0, main));
-    if (rest) TRY(wait(main, ss->done));
-    rest = false;
-    // the next block column: W[k1:, k1:k2] -= P P[:128]^T
-    TRY(trnblas_hip_dgemm(0, 1, rows, kNB, kNB, -1.0, L + k1 * npad + k0, npad, 0,
-                          L + k1 * npad + k0, npad, 0, 1.0, W + k1 * npad + k1, npad, 0,
-                          W + k1 * npad + k1, npad, 0, 1, 0, 0, main));
-    // one event for both: the side stream's trailing update and the
-    // inverse stream's block row (one record per step fewer on the host)
-    if (k2 < npad || b > 0) TRY(record(ss->ready, main));
-    TRY(inv_row());
-    if (k2 < npad) {
-      const int64_t r2 = npad - k2;
+    if (k2 < npad) {  // the next step's columns
+      if (rest) TRY(wait(main, ss->done));
+      rest = false;
       const double* R = L + k2 * npad + k0;
-      double* Wt = W + k2 * npad + k2;
+      TRY(mm(true, npad - k2, k3 - k2, k2 - k0, -1.0, R, R, npad, 1.0, W + k2 * npad + k2, npad, 0, 0,
+             main));
+    }
+    // one event for both: the side stream's trailing update and the
+    // inverse stream's rows
+    if (inv != main) TRY(record(ss->ready, main));
+    if (k3 < npad) {
+      const double* R = L + k3 * npad + k0;
       TRY(wait(ss->side, ss->ready));
-      TRY(trnblas_hip_dgemm(0, 1, r2, r2, kNB, -1.0, R, npad, 0, R, npad, 0, 1.0, Wt, npad, 0, Wt,
-                            npad, 0, 1, 1, 0, ss->side));
+      TRY(mm(true, npad - k3, npad - k3, k2 - k0, -1.0, R, R, npad, 1.0, W + k3 * npad + k3, npad, 1,
+             0, ss->side));
       TRY(record(ss->done, ss->side));
       rest = true;
     }
+    if (inv != main) TRY(wait(inv, ss->ready));
+    if (k2 > k1) {  // Y_10 = -Y_11 (L_10 Y_00)
+      TRY(mm(false, kNB, kNB, kNB, 1.0, L + k1 * npad + k0, Y00, npad, 0.0, S, kNB, 0,
+             TRNBLAS_TRI_B_LOWER, inv));
+      TRY(mm(false, kNB, kNB, kNB, -1.0, Y11, S, kNB, 0.0, Y + k1 * npad + k0, npad, 0,
+             TRNBLAS_TRI_A_LOWER, inv));
+    }
+    if (k0 > 0)  // Y[B, :k0] = -Y_BB T
+      TRY(mm(false, k2 - k0, k0, k2 - k0, -1.0, Y00, T, npad, 0.0, Y + k0 * npad, npad, 0,
+             TRNBLAS_TRI_A_LOWER, inv));
+    if (k2 < npad)  // T = L[B', :k2] Y[:k2, :k2] of the next rows B'
+      TRY(mm(false, k3 - k2, k2, k2, 1.0, L + k2 * npad, Y, npad, 0.0, T, npad, 0,
+             TRNBLAS_TRI_B_LOWER, inv));
   }
-  if (rest) TRY(wait(main, ss->done));
-  if (inv) {
-    TRY(record(ss->inverted, ss->inv));
+  if (inv != main) {
+    TRY(record(ss->inverted, inv));
     TRY(wait(main, ss->inverted));
   }
   const unsigned tb = (unsigned)((n + 63) / 64);

@@ -651,9 +651,9 @@ def metric_inv_half(J: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         raise ValueError("metric_inv_half: J must be a square float64 matrix")
     n = J.shape[0]
     X = torch.empty((n, n), dtype=torch.float64, device=dev)
-    info = torch.zeros(1, dtype=torch.int32, device=dev)
     if n == 0:
-        return X, info
+        return X, torch.zeros(1, dtype=torch.int32, device=dev)
+    info = torch.empty(1, dtype=torch.int32, device=dev)  # (cleared by the driver)
     if J.stride(1) != 1 or J.stride(0) < n:
         J = J.contiguous()
     lib = _lib.load()
