@@ -269,3 +269,20 @@ def test_pair_energy_wide_range_rows(dev, math, tol):
     rel = abs(got - want) / abs(want)
     print(f"wide-range rows, {math}: rel {rel:.2e}", flush=True)
     assert rel <= tol, rel
+
+
+@pytest.mark.parametrize("nocc,nvir,naux", [(1, 5, 3), (3, 97, 33), (10, 96, 64), (31, 95, 40), (32, 60, 70), (33, 90, 64),
+                                            (22, 100, 65)])
+def test_pair_energy_walks_agree(dev, nocc, nvir, naux):
+    # the implicit walk goes pair by pair or by squares of pairs depending on
+    # the item count (512 on 256 CUs: 31, 32 rows of one tile pair on either
+    # side, 22 x 3 tile pairs past it); its total is the sum of the explicit
+    # pairs' energies (the same kernel's, or the same sums) to fp64 rounding
+    from trnblas_amd.hip import kernels
+
+    B, eo, ev = (x.to(dev) for x in _inputs(nocc, nvir, naux, 7))
+    got = float(kernels.pair_energy_sym(B, eo, ev, math="fp16x3"))
+    i, j = torch.triu_indices(nocc, nocc)
+    e = kernels.pair_energies(B, B, eo, eo, ev, i.int(), j.int(), math="fp16x3").cpu()
+    want = float((e * torch.where(i == j, 1.0, 2.0)).sum())
+    assert abs(got - want) <= 1e-13 * abs(want)

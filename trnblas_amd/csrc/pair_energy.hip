@@ -297,8 +297,11 @@ __global__ __launch_bounds__(256) void zero_f64_kernel(double* p, int64_t n) {
   if (i < n) p[i] = 0.0;
 }
 
-__global__ __launch_bounds__(1024) void pair_total_kernel(const double* e_pair, int npairs,
-                                                          int nocc, const int32_t* pair_i,
+// With `partial` the pairs' energies are summed here from their nq partials,
+// in pair_sum_kernel's order (few partials: one launch instead of two).
+__global__ __launch_bounds__(1024) void pair_total_kernel(const double* e_pair,
+                                                          const double* partial, int nq,
+                                                          int npairs, int nocc, const int32_t* pair_i,
                                                           const int32_t* pair_j,
                                                           const double* pair_w, double* total) {
   __shared__ double red[16];
@@ -313,7 +316,14 @@ __global__ __launch_bounds__(1024) void pair_total_kernel(const double* e_pair, 
       tri_pair(p, nocc, i, j);
       w = i == j ? 1.0 : 2.0;
     }
-    s += w * e_pair[p];
+    double e;
+    if (partial) {
+      e = 0.0;
+      for (int q = 0; q < nq; ++q) e += partial[(int64_t)p * nq + q];
+    } else {
+      e = e_pair[p];
+    }
+    s += w * e;
   }
   s = wave_sum(s);
   if ((tid & 63) == 0) red[tid >> 6] = s;
@@ -1578,12 +1588,18 @@ static void x3_split(const float* X, int64_t n, int64_t ld_occ, int64_t ld_vir, 
                        (int)threads, X, ld_occ, ld_vir, P);
 }
 
+// The implicit fp16x3 walk goes pair by pair (pair_energy_x3_kernel, the same
+// sums) while its items all fit the chip at two workgroups per CU: the
+// squares would leave most CUs idle, each with four pairs' work to do. Call
+// in us, pairs / squares: 10 x 43 x 1262 45.9 / 74.2, 16 x 112 x 384 42.6 /
+// 49.6 (408 items), 7 x 458 x 405 57.4 / 58.7 (420); past two per CU 32 x 92 x
+// 1314 107 / 90 (528), 8 x 495 x 444 92 / 66 (756).
 template <int NPC>
 static void split_launch(const PairArgs& g, bool implicit, int64_t citems, int64_t items,
                          hipStream_t s) {
-  if (implicit && NPC == 2)
+  if (implicit && NPC == 2 && items > 2 * device_cus())
     hipLaunchKernelGGL(pair_energy_quad_kernel, dim3((unsigned)citems), dim3(512), 0, s, g);
-  else if (implicit)
+  else if (implicit && NPC == 3)
     hipLaunchKernelGGL(pair_energy_x3c_kernel<3>, dim3((unsigned)citems), dim3(512), 0, s, g);
   else
     hipLaunchKernelGGL(pair_energy_x3_kernel<NPC>, dim3((unsigned)items), dim3(256), 0, s, g);
@@ -1715,13 +1731,18 @@ static int pair_energy_run(int npc, const char* name, int64_t nvir, int64_t naux
   }
   int rc = check_launch(name);
   if (rc) return rc;
-  hipLaunchKernelGGL(pair_sum_kernel, dim3((unsigned)((npairs + 255) / 256)), dim3(256), 0, s,
-                     (const double*)g.partial, (int)npairs, (int)nq, e_pair);
-  rc = check_launch(name);
-  if (rc) return rc;
+  // the per-pair sums on their own unless only a total of few partials is asked
+  const bool total_only = out_pairs == nullptr && out_total != nullptr && items <= 8192;
+  if (!total_only) {
+    hipLaunchKernelGGL(pair_sum_kernel, dim3((unsigned)((npairs + 255) / 256)), dim3(256), 0, s,
+                       (const double*)g.partial, (int)npairs, (int)nq, e_pair);
+    rc = check_launch(name);
+    if (rc) return rc;
+  }
   if (out_total) {
     hipLaunchKernelGGL(pair_total_kernel, dim3(1), dim3(1024), 0, s, (const double*)e_pair,
-                       (int)npairs, (int)nocc, pair_i, pair_j, pair_w, out_total);
+                       total_only ? (const double*)g.partial : nullptr, (int)nq, (int)npairs,
+                       (int)nocc, pair_i, pair_j, pair_w, out_total);
     rc = check_launch(name);
   }
   return rc;
