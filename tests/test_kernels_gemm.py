@@ -630,3 +630,27 @@ def test_sgemm_any_alignment(dev, M, N, K, batch, ta, tb):
     ref = 1.5 * (Ad @ Bd) - 0.5 * C.double()
     den = 1.5 * (Ad.abs() @ Bd.abs()) + 0.5 * C.double().abs()
     assert ((D.double() - ref).abs() / den).max().item() <= 1e-6
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0**-8), (torch.float16, 2.0**-10)])
+@pytest.mark.parametrize("M,N,K,batch", [(8, 8, 8, 1), (128, 136, 64, 1), (264, 120, 136, 1), (504, 496, 192, 1),
+                                         (256, 128, 320, 40), (1784, 2032, 264, 1)])
+def test_one_round_16bit(dev, dtype, tol, M, N, K, batch, ta, tb):
+    # hgemm128_kernel (up to one 128 x 128 tile per CU): 1..6 k-tiles against its
+    # four LDS stages, ragged tile edges and K tails, batches, against fp64 at
+    # the 16-bit gate (one rounding of |A||B| + |C|)
+    from trnblas_amd.hip import kernels
+
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(batch, *((K, M) if ta else (M, K)), generator=g).to(dtype)
+    B = torch.randn(batch, *((N, K) if tb else (K, N)), generator=g).to(dtype)
+    C = torch.randn(batch, M, N, generator=g).to(dtype)
+    a, b = (A.mT if ta else A), (B.mT if tb else B)
+    if batch == 1:
+        D = kernels.gemm(a[0].to(dev), b[0].to(dev), 1.0, 0.5, C[0].to(dev))[None].cpu()
+    else:
+        D = kernels.gemm(a.to(dev), b.to(dev), 1.0, 0.5, C.to(dev)).cpu()
+    ref = a.double() @ b.double().contiguous() + 0.5 * C.double()
+    den = a.double().abs() @ b.double().abs().contiguous() + 0.5 * C.double().abs()
+    assert ((D.double() - ref).abs() / den).max().item() <= tol

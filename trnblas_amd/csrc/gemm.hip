@@ -910,6 +910,166 @@ __global__ __launch_bounds__(512, 1) void hgemm256_kernel(GemmArgs g) {
   store_tile<T, false, FM, FN, BM, BN>(g, acc, bat, m0, n0, wm0, wn0, lane, -1, 0);
 }
 
+// 16-bit GEMM on 128 x 128 tiles, one workgroup per CU: eight compute waves
+// (64 x 32 each, 2 x 1 blocks of MFMA 32x32x16) and four movers in the manner of
+// sgemm_pipe_kernel: k-tiles of 64 go into the movers' registers two k-tiles
+// ahead and from there into four LDS stages of 32 KiB, and the barrier that
+// publishes k-tile t + 1 comes before the last chunk's MFMAs of t. LDS layout,
+// swizzles and fragment reads are gemm_dma_kernel's. About 0.65 us per k-tile
+// (the LDS moves 128 KiB in it) and 6 us besides, whatever the tiles; four
+// compute waves of 64 x 64, LDS DMA by the compute waves (1 us per k-tile: a
+// wave's DMAs complete one at a time) and four register sets per mover (no
+// change) were measured too.
+constexpr int kHCompute = 8;
+template <typename T, bool AKC, bool BKC>
+__global__ __launch_bounds__(64 * (kHCompute + 4), 1) void hgemm128_kernel(GemmArgs g) {
+  static_assert(sizeof(T) == 2, "16-bit operands");
+  constexpr int EV = 8, BM = 128, BK = 64, FM = 2, FN = 8 / kHCompute, CH = 2 * EV;
+  constexpr int PANEL = BM * BK, MG = BM / EV, NS = 4;
+  __shared__ __attribute__((aligned(16))) T lds[NS][2 * PANEL];
+
+  const int tid = threadIdx.x;
+  int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int M = g.M, N = g.N, K = g.K, nk = g.nk;
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  int bat, tm, tn;
+  decode_tile<false>(g, t, bat, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BM;
+
+  if (wave >= kHCompute) {
+    const int m = wave - kHCompute;
+    const bool onB = m >= 2;
+    const bool kc = onB ? BKC : AKC;
+    const T* X = static_cast<const T*>(onB ? g.B : g.A) + bat * (onB ? g.sB : g.sA);
+    const int64_t ld = onB ? g.ldb : g.lda;
+    const int r0 = onB ? n0 : m0, left = (onB ? N : M) - r0;
+    // block b = 8 (m & 1) + u of the panel (1 KiB): lane l's group lands at
+    // byte 16 l. kq: k past the lane's group (it is inside while kq <= k left)
+    uint32_t v[8];
+    int kq[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int b = 8 * (m & 1) + u;
+      int row, grp;
+      if (kc) {
+        row = 8 * b + (lane >> 3);
+        grp = (lane & 7) ^ ((row >> 1) & 7);
+        kq[u] = row < left ? EV * grp + 1 : 1 << 30;
+      } else {
+        row = (64 / MG) * b + lane / MG;
+        grp = (lane % MG) ^ (4 * (row & 3));
+        kq[u] = EV * grp < left ? row + 1 : 1 << 30;
+      }
+      v[u] = (uint32_t)((int64_t)row * ld * (int64_t)sizeof(T) + 16 * grp);
+    }
+    auto gload = [&](int kt, i32x4(&r)[8]) __attribute__((always_inline)) {
+      const int k0 = kt * BK, kl = K - k0;
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(kc ? X + r0 * ld + k0 : X + (int64_t)k0 * ld + r0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        r[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, kq[u] <= kl ? v[u] : kOob, 0, 0);
+    };
+    auto lwrite = [&](int kt, const i32x4(&r)[8]) __attribute__((always_inline)) {
+      T* dst = lds[kt & (NS - 1)] + (onB ? PANEL : 0) + 8 * (m & 1) * 512 + 8 * lane;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) *reinterpret_cast<i32x4*>(dst + u * 512) = r[u];
+    };
+    if (nk == 0) return;
+    // (the barriers and register sets of sgemm_pipe_kernel's movers)
+    i32x4 ra[8], rb[8];
+    gload(0, ra);
+    if (nk > 1) gload(1, rb);
+    lwrite(0, ra);
+    if (nk > 2) gload(2, ra);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    auto step = [&](int s, i32x4(&r)[8]) __attribute__((always_inline)) {
+      lwrite(s + 1, r);
+      if (s + 3 < nk) gload(s + 3, r);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    int s = 0;
+    for (; s + 2 < nk; s += 2) {
+      step(s, rb);
+      step(s + 1, ra);
+    }
+    if (s + 1 < nk) step(s, rb);
+    return;
+  }
+
+  const int wm0 = (wave & 1) * 64, wn0 = (wave >> 1) * 32 * FN;
+  auto frag = [&](const T* p, bool kc, int r, int kk) __attribute__((always_inline)) {
+    if (kc)
+      return *reinterpret_cast<const i32x4*>(p + r * BK + EV * ((kk / EV) ^ ((r >> 1) & 7)));
+    const int i = lane & 15;
+    const int c0 = r - i + 4 * (i & 3);
+    const int k1 = kk + (i >> 2);
+    const T* s0 = p + k1 * BM + EV * ((c0 / EV) ^ (4 * (k1 & 3))) + (c0 & 4);
+    union {
+      s16x4 h[2];
+      i32x4 v;
+    } u;
+    u.h[0] = lds_tr16(s0);
+    u.h[1] = lds_tr16(s0 + 4 * BM);
+    return u.v;
+  };
+  f32x16 acc[FM][FN], sum[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = sum[i][j][r] = 0.0f;
+  i32x4 fa[2][FM], fb[2][FN];
+  auto rd = [&](const T* cur, int c, int set) __attribute__((always_inline)) {
+    const int kk = c * CH + (lane >> 5) * EV;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) fa[set][i] = frag(cur, AKC, wm0 + i * 32 + (lane & 31), kk);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) fb[set][j] = frag(cur + PANEL, BKC, wn0 + j * 32 + (lane & 31), kk);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto mm = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) mma_frag(acc[i][j], fa[set][i], fb[set][j], (T*)nullptr);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (nk > 0) {
+    asm volatile("s_barrier" ::: "memory");  // k-tile 0 is in LDS
+    rd(lds[0], 0, 0);
+    int chain = g.span;
+    for (int kt = 0; kt < nk; ++kt) {
+      asm volatile("" : "+v"(lane));
+      const T* cur = lds[kt & (NS - 1)];
+      rd(cur, 1, 1);
+      mm(0);
+      rd(cur, 2, 0);
+      mm(1);
+      rd(cur, 3, 1);
+      mm(0);
+      if (kt + 1 < nk) {
+        asm volatile("s_barrier" ::: "memory");
+        rd(lds[(kt + 1) & (NS - 1)], 0, 0);
+      }
+      mm(1);
+      if (--chain == 0) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) fold_span(sum[i][j], acc[i][j]);
+        chain = g.span;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) fold_span(sum[i][j], acc[i][j]);
+  }
+  store_tile<T, false, FM, FN, BM, BM>(g, sum, bat, m0, n0, wm0, wn0, lane, -1, 0);
+}
+
 // Sums the stream-K partials of each split tile in workgroup order
 // (deterministic) and applies the epilogue. Grid: (split tiles, BM / 8):
 // each workgroup finishes 8 rows of one tile, one float4 of partials per
@@ -1355,6 +1515,29 @@ static int launch_wide(GemmArgs g, hipStream_t s) {
   return check_launch("trnblas_hip_gemm");
 }
 
+// hgemm128_kernel for up to one 128 x 128 tile per CU, unless enough k-tiles
+// let gemm_dma_kernel's narrow tiles / stream-K split them better: few tiles,
+// by the two kernels' times (about 6 + 0.62 nk us against 12 + 0.004 nk tiles
+// from 20 k-tiles on), or a round that narrow tiles fill as well. Measured
+// (bf16, us, NN, against gemm_dma_kernel): 504 x 496 x 512 10.4 / 11.9, 1016 x
+// 1008 x 1024 15.6 / 20.5, 1784 x 2032 x 2048 28.5 / 60.5, 2048^2 x 1024 18.3 /
+// 29.9, 64 x (256^2 x 1024) 19.7 / 30.5; left to it: 504 x 496 x 2048 (24.1) /
+// 16.7, 1016 x 1008 x 2048 (25.4) / 20.6, 2048^3 (30.5) / 30.5.
+static bool one_round_pays(const GemmArgs& g) {
+  const double t = g.ntiles, cus = device_cus(), nk = g.nk;
+  if (t > cus) return false;
+  if (t < cus / 8) return nk < 16;
+  if (nk >= 20 && nk * (0.62 - 1.024 * t / cus) > 6.0) return false;
+  return t < 0.9 * cus || nk < 24;
+}
+
+template <typename T, bool AKC, bool BKC>
+static int launch_one_round(const GemmArgs& g, hipStream_t s) {
+  hipLaunchKernelGGL((hgemm128_kernel<T, AKC, BKC>), dim3(g.ntiles), dim3(64 * (kHCompute + 4)), 0, s,
+                     g);
+  return check_launch("trnblas_hip_gemm");
+}
+
 template <typename T, bool AKC, bool BKC, bool VEC, bool SYRK>
 static int launch_t(GemmArgs g, size_t ws_bytes, hipStream_t s) {
   using C = Cfg<T>;
@@ -1369,6 +1552,7 @@ static int launch_t(GemmArgs g, size_t ws_bytes, hipStream_t s) {
     const int64_t span_a = (AKC ? 256 : 64) * g.lda * 2, span_b = (BKC ? 256 : 64) * g.ldb * 2;
     if (wide_tiles_pay(g) && span_a < (int64_t)kRecords - 64 && span_b < (int64_t)kRecords - 64)
       return launch_wide<T, AKC, BKC>(g, s);
+    if (one_round_pays(g)) return launch_one_round<T, AKC, BKC>(g, s);
   }
   if constexpr (DMA && !SYRK) {
     if (narrow_tiles_pay(g, (int)sizeof(T))) return launch_narrow<T, AKC, BKC>(g, ws_bytes, s);
