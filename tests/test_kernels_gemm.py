@@ -654,3 +654,67 @@ def test_one_round_16bit(dev, dtype, tol, M, N, K, batch, ta, tb):
     ref = a.double() @ b.double().contiguous() + 0.5 * C.double()
     den = a.double().abs() @ b.double().abs().contiguous() + 0.5 * C.double().abs()
     assert ((D.double() - ref).abs() / den).max().item() <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize(
+    "M,N,K,batch",
+    # 16-bit 32 x 32 kernel, K split over 4 and 8 waves: one off its tile and its
+    # 32-wide chunks, single rows, columns and k, odd last pairs, more chunks than
+    # waves, and aligned products that it serves
+    [(1, 1, 1, 1), (3, 1, 2, 1), (1, 33, 31, 1), (33, 31, 33, 1), (35, 65, 257, 3), (31, 97, 2049, 1),
+     (129, 130, 65, 5), (255, 257, 127, 1), (96, 64, 128, 1), (384, 384, 384, 1)],
+)  # fmt: skip
+def test_hgemm_any_alignment(dev, M, N, K, batch, ta, tb, dtype):
+    # in place on ragged operands whose neighbours hold NaN, against fp64: fp32
+    # sums (1e-6 |A||B| + |C|) and one rounding to the output type
+    from trnblas_amd.hip import kernels
+
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 7 * K)
+
+    def operand(r, c):  # a (batch, r, c) view inside a NaN-filled buffer; odd leading dimension unless c % 32 == 0
+        full = torch.full((batch, r, c + (8 if c % 32 == 0 else 3)), float("nan"), device=dev, dtype=dtype)
+        full[:, :, :c] = torch.randn(batch, r, c, generator=g, device=dev)
+        return full[:, :, :c]
+
+    A = operand(K, M).mT if ta else operand(M, K)
+    B = operand(N, K).mT if tb else operand(K, N)
+    C = operand(M, N)
+    D = kernels.gemm(A[0], B[0], 1.5, -0.5, C[0])[None] if batch == 1 else kernels.gemm(A, B, 1.5, -0.5, C)
+    Ad, Bd = A.double().contiguous(), B.double().contiguous()
+    ref = 1.5 * (Ad @ Bd) - 0.5 * C.double()
+    den = 1.5 * (Ad.abs() @ Bd.abs()) + 0.5 * C.double().abs()
+    eps = torch.finfo(dtype).eps
+    tiny = torch.finfo(dtype).tiny * torch.finfo(dtype).eps  # the rounding of results below the normal range
+    assert ((D.double() - ref).abs() <= 0.5 * eps * ref.abs() + (1 + eps) * 1e-6 * den + tiny).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("uplo", ["lower", "upper"])
+@pytest.mark.parametrize("n,k", [(1, 1), (2, 3), (31, 33), (33, 31), (65, 257), (98, 231), (130, 1025), (257, 64), (160, 320)])
+def test_syrk_small_tiles(dev, n, k, uplo, trans, dtype):
+    # SYRK on the 32 x 32 kernels: both triangles bit-equal, only the referenced
+    # triangle of C read (NaN in the other one), NaN beside the operand, against fp64
+    from trnblas_amd.hip import kernels
+
+    g = torch.Generator(device=dev).manual_seed(n + 5 * k)
+    r, c = (k, n) if trans else (n, k)
+    full = torch.full((r, c + (8 if c % 32 == 0 else 3)), float("nan"), device=dev, dtype=dtype)
+    full[:, :c] = torch.randn(r, c, generator=g, device=dev)
+    A = full[:, :c]
+    X = torch.randn(n, n, generator=g, device=dev).to(dtype)
+    Cs = (torch.tril(X) + torch.tril(X, -1).mT).double()
+    nan = torch.full_like(X, float("nan"))
+    tri = torch.ones(n, n, device=dev, dtype=torch.bool)
+    tri = torch.tril(tri) if uplo == "lower" else torch.triu(tri)
+    C = torch.where(tri, Cs.to(dtype), nan)
+    D = kernels.syrk(A, 1.5, -0.5, C, trans=trans, uplo=uplo)
+    assert torch.equal(D, D.mT)
+    Ad = (A.mT if trans else A).double()
+    ref = 1.5 * (Ad @ Ad.mT) - 0.5 * Cs
+    den = 1.5 * (Ad.abs() @ Ad.abs().mT) + 0.5 * Cs.abs()
+    eps = 0.0 if dtype == torch.float32 else torch.finfo(dtype).eps
+    tiny = torch.finfo(dtype).tiny * torch.finfo(dtype).eps
+    assert ((D.double() - ref).abs() <= 0.5 * eps * ref.abs() + (1 + eps) * 1e-6 * den + tiny).all()

@@ -128,48 +128,6 @@ __device__ __forceinline__ i32x4 read_frag(const T* buf, int row, int kk) {
   }
 }
 
-// Lower-triangle tile t -> (tm, tn), tm >= tn, of a triangle T tiles on a
-// side, in groups of 8 tile rows: group G (rows 8G .. 8G + R - 1, R = 8 but
-// for the last) lists its whole columns tn < 8G (R tiles each, top to
-// bottom), then its own R-row triangle column by column; groups start at
-// tile 32 G^2 + 4 G. Consecutive tiles (one XCD's share of a round) then
-// cover an 8-row, 8-column block of operand panels (13-20 distinct panels per
-// 64 tiles of a 32-tile side, against ~35 for a row-major walk).
-__device__ __forceinline__ void tri_tile(int t, int T, int& tm, int& tn) {
-  int G = (int)((sqrtf(16.0f + 128.0f * (float)t) - 4.0f) * (1.0f / 64.0f));
-  while (G > 0 && 32 * G * G + 4 * G > t) --G;
-  while ((G + 1) * 8 < T && 32 * (G + 1) * (G + 1) + 4 * (G + 1) <= t) ++G;
-  int u = t - (32 * G * G + 4 * G);
-  const int R = min(8, T - 8 * G);
-  if (u < 8 * G * R) {
-    tm = 8 * G + u % R;
-    tn = u / R;
-    return;
-  }
-  u -= 8 * G * R;
-  int c = 0;
-  while (u >= R - c) {
-    u -= R - c;
-    ++c;
-  }
-  tm = 8 * G + c + u;
-  tn = 8 * G + c;
-}
-
-// SYRK: whether the upper triangle of C is the one referenced: g.uplo, or,
-// with triangle flags (flags[0]: the strict upper triangle holds a nonzero,
-// flags[1]: the strict lower one), the other triangle when only that one
-// holds off-diagonal entries (the rule of trnblas/level3.py:305-329, decided
-// on the device so the host need not wait for the flags before the launch).
-__device__ __forceinline__ int syrk_upper(const GemmArgs& g) {
-  int up = g.uplo;
-  if (g.tri != nullptr) {
-    const int has_up = g.tri[0], has_lo = g.tri[1];
-    if (up ? (has_lo && !has_up) : (has_up && !has_lo)) up ^= 1;
-  }
-  return up;
-}
-
 // D = alpha acc + beta C for one output element (C not read when beta == 0);
 // SYRK: m >= n only, written to both triangles, C read from the side `up`
 // (syrk_upper).
@@ -1579,12 +1537,17 @@ static int launch_dtype(const GemmArgs& g, bool akc, bool bkc, bool vec, size_t 
                         hipStream_t s) {
   // fp32 GEMM: sgemm.hip's kernels take every unaligned product and the
   // aligned ones that they serve better (sgemm_launch), but not the shapes of
-  // sgemm_pipe_kernel (C1: 137 us against 145 on 64 x 64 tiles)
+  // sgemm_pipe_kernel (C1: 137 us against 145 on 64 x 64 tiles). Small SYRKs
+  // and 16-bit products go to 32 x 32 tiles (ssyrk_launch, hgemm_launch).
   constexpr bool kF32Gemm = !SYRK && sizeof(T) == 4;
+  int rc = TRNBLAS_OK;
   if constexpr (kF32Gemm) {
-    int rc = TRNBLAS_OK;
     if (!(vec && !akc && !bkc && pipe_pays(g)) && sgemm_launch(g, akc, bkc, vec, ws_bytes, s, &rc))
       return rc;
+  } else if constexpr (sizeof(T) == 4) {
+    if (ssyrk_launch(g, akc, vec, s, &rc)) return rc;
+  } else {
+    if (hgemm_launch<T, SYRK>(g, akc, bkc, vec, s, &rc)) return rc;
   }
 #define TRNBLAS_L(a, b, v)                               \
   if constexpr (v || !kF32Gemm) {                        \
