@@ -584,3 +584,35 @@ def test_ozaki_plan_known_answers():
     mbs, kbs, nbs = ozaki.plan(2304, 512, 1500, 3, 2 * 3 * 512 * 1024)
     assert len(mbs) > 1 and len(nbs) > 1 and len(kbs) == 1
     assert len(ozaki.plan(128, 3072, 20, 8, 2 * 8 * 128 * 1024)[1]) > 1
+
+
+@pytest.mark.parametrize("dtype,shape,packs", [
+    (torch.bfloat16, (1023, 1023, 1023), False), (torch.bfloat16, (1025, 1025, 1025), True),  # 2^30, few tiles
+    (torch.bfloat16, (3201, 1025, 99), True),  # more than 12 tiles per CU, 2^28
+    (torch.float32, (1023, 1023, 1027), False),
+])  # fmt: skip
+def test_unaligned_gemm_packing_starts_later_on_small_grids(monkeypatch, dtype, shape, packs):
+    # sizes only: the operands are expanded scalars, and packing is recorded
+    from trnblas_amd.hip import kernels as k
+
+    seen = []
+    monkeypatch.setattr(k, "_pack_k", lambda X, kp: seen.append(kp) or X)
+    M, N, K = shape
+    A, B = torch.zeros(1, dtype=dtype).expand(M, K), torch.zeros(1, dtype=dtype).expand(K, N)
+    k._packed_operands(A, B, A, False, K, 0, B, False, N, 0, M, N, K, 1)
+    assert bool(seen) == packs
+
+
+@pytest.mark.parametrize("dtype,n,kk,packs", [
+    (torch.float32, 1025, 2049, False), (torch.float32, 2049, 1025, True), (torch.float32, 517, 4099, True),
+    (torch.bfloat16, 1025, 333, False), (torch.bfloat16, 1025, 1025, True), (torch.bfloat16, 2231, 89, True),
+    (torch.bfloat16, 365, 2049, True),
+])  # fmt: skip
+def test_unaligned_syrk_packing_starts_later_on_small_grids(monkeypatch, dtype, n, kk, packs):
+    from trnblas_amd.hip import kernels as k
+
+    seen = []
+    monkeypatch.setattr(k, "_pack_k", lambda X, kp: seen.append(kp) or X)
+    A = torch.zeros(1, dtype=dtype).expand(n, kk)
+    k._packed_syrk_operand(A, False, A, False, kk, n, kk)
+    assert bool(seen) == packs

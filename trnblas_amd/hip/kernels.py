@@ -96,20 +96,29 @@ def _batched_layout(X: torch.Tensor):
 # 16-byte aligned base, and a leading dimension, batch stride and contiguous
 # extent that are multiples of 16 bytes. Other operands run on
 # register-staged kernels: fp32 GEMM at any alignment on sgemm.hip's (72-125
-# TFLOP/s from 1535^3 up), the rest at 74 TFLOP/s fp32 SYRK and 81 TFLOP/s
+# TFLOP/s from 1535^3 up), small 16-bit products and SYRKs on 32 x 32 tiles
+# (hgemm.hip, sgemm.hip), the rest at 74 TFLOP/s fp32 SYRK and 81 TFLOP/s
 # bf16 at 4095^3 (737 after packing). From PACK_MIN_MACS multiply-adds per
 # launch on, such operands are first copied by trnblas_hip_pack_k into fresh
 # K-contiguous buffers whose rows are padded with zeros to a multiple of 16
 # bytes (zero products add nothing to any sum; the reference pads its kernel
 # operands the same way, nki/dispatch.py:2344-2368) and the product takes the
-# DMA kernel. Below it the pack launches cost more than they save (bf16 511^3
-# 29 us in place, 32 packed; 767^3 38 and 34). An fp32 GEMM, whose kernels read
-# any alignment, packs from F32_GEMM_PACK_FACTOR times that size: over random
+# DMA kernel. Below it the pack launches cost more than they save. Where the
+# 32 x 32 kernels serve unaligned operands (DIRECT_TILES), packing starts at 4
+# times that size: over random shapes there they are 2.0x faster (batched bf16,
+# even from 2^30 on: 31 x (175 x 164 x 1098) 41 us packed, 20 in place), 1.4x
+# (fp32 SYRK, none slower; 879 x 2372 47 and 37) and 1.4x (16-bit SYRK; past its
+# limits packed is up to 1.3x faster, 2230 x 89 13 us against 16). An
+# fp32 GEMM, whose kernels read any alignment, packs from F32_GEMM_PACK_FACTOR times that size: over random
 # unaligned shapes packing is 1.6x slower than in place at 2^30 multiply-adds,
 # 1.26x at 2^33, 1.12x at 2^36, where cubes are even (4095^3 1100 us packed,
 # 1186 in place).
 PACK_MIN_MACS = {4: 1 << 30, 2: 1 << 28}
 F32_GEMM_PACK_FACTOR = 64
+# Largest numbers of 32 x 32 tiles (per launch, 256 CUs) of the unaligned 16-bit
+# GEMMs and the fp32 / 16-bit SYRKs that are packed only later, and the largest
+# k of those SYRKs
+DIRECT_TILES = {"gemm": 12 * 256, "syrk": {4: (20 * 256, 4096), 2: (4 * 256, 2048)}}
 
 # TRNBLAS_GEMM_RAGGED=0 restores the reference's pad-first path
 # (nki/dispatch.py:144-151, read at import as there): every operand the DMA
@@ -150,7 +159,10 @@ def _packed_operands(A, B, a, ta, lda, sa, b, tb, ldb, sb, M, N, K, nb):
     with the operands the DMA kernel cannot read packed K-contiguous (and K
     padded when it is not a multiple of 16 bytes)."""
     ev = 16 // A.element_size()
-    if nb * M * N * K < _pack_min_macs(A.element_size()) or M == 0 or N == 0 or K == 0:
+    least = _pack_min_macs(A.element_size())
+    if ev == 8 and nb * -(-M // 32) * -(-N // 32) <= DIRECT_TILES["gemm"]:
+        least *= 4
+    if nb * M * N * K < least or M == 0 or N == 0 or K == 0:
         return a, ta, lda, sa, b, tb, ldb, sb, K
     a_ok = _dma_ready(a, lda, sa, M if ta else K, ev)
     b_ok = _dma_ready(b, ldb, sb, K if tb else N, ev)
@@ -170,7 +182,11 @@ def _packed_syrk_operand(A, trans, a, t, lda, n, k):
     """SYRK's (a, t, lda, k) for op(A) (n, k): as laid out, or packed
     K-contiguous with k padded to a multiple of 16 bytes (see _packed_operands)."""
     ev = 16 // A.element_size()
-    if n * n * k < _pack_min_macs(A.element_size(), True) or n == 0 or k == 0 or _dma_ready(a, lda, 0, n if t else k, ev):
+    least, tiles = _pack_min_macs(A.element_size(), True), -(-n // 32)
+    most, longest = DIRECT_TILES["syrk"][A.element_size()]
+    if tiles * (tiles + 1) // 2 <= most and k <= longest:
+        least *= 4
+    if n * n * k < least or n == 0 or k == 0 or _dma_ready(a, lda, 0, n if t else k, ev):
         return a, t, lda, k
     kp = -(-k // ev) * ev
     return _pack_k(A.t() if trans else A, kp), False, kp, kp
