@@ -603,16 +603,18 @@ def test_unaligned_gemm_packing_starts_later_on_small_grids(monkeypatch, dtype, 
     assert bool(seen) == packs
 
 
-@pytest.mark.parametrize("dtype,n,kk,packs", [
-    (torch.float32, 1025, 2049, False), (torch.float32, 2049, 1025, True), (torch.float32, 517, 4099, True),
-    (torch.bfloat16, 1025, 333, False), (torch.bfloat16, 1025, 1025, True), (torch.bfloat16, 2231, 89, True),
-    (torch.bfloat16, 365, 2049, True),
+@pytest.mark.parametrize("dtype,n,kk,trans,packs", [
+    (torch.float32, 1025, 2049, False, False), (torch.float32, 1025, 2048, True, False),
+    (torch.float32, 2049, 1025, False, True), (torch.float32, 517, 4099, False, True),
+    (torch.bfloat16, 1025, 333, True, False), (torch.bfloat16, 1025, 333, False, True),
+    (torch.bfloat16, 1025, 1025, True, True), (torch.bfloat16, 2231, 89, True, True),
+    (torch.bfloat16, 365, 2049, True, True),
 ])  # fmt: skip
-def test_unaligned_syrk_packing_starts_later_on_small_grids(monkeypatch, dtype, n, kk, packs):
+def test_unaligned_syrk_packing_starts_later_on_small_grids(monkeypatch, dtype, n, kk, trans, packs):
     from trnblas_amd.hip import kernels as k
 
     seen = []
     monkeypatch.setattr(k, "_pack_k", lambda X, kp: seen.append(kp) or X)
-    A = torch.zeros(1, dtype=dtype).expand(n, kk)
-    k._packed_syrk_operand(A, False, A, False, kk, n, kk)
+    A = torch.zeros(1, dtype=dtype).expand(*((kk, n) if trans else (n, kk)))
+    k._packed_syrk_operand(A, trans, A, trans, A.shape[1], n, kk)
     assert bool(seen) == packs

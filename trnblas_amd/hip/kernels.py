@@ -105,19 +105,21 @@ def _batched_layout(X: torch.Tensor):
 # operands the same way, nki/dispatch.py:2344-2368) and the product takes the
 # DMA kernel. Below it the pack launches cost more than they save. Where the
 # 32 x 32 kernels serve unaligned operands (DIRECT_TILES), packing starts at 4
-# times that size: over random shapes there they are 2.0x faster (batched bf16,
-# even from 2^30 on: 31 x (175 x 164 x 1098) 41 us packed, 20 in place), 1.4x
-# (fp32 SYRK, none slower; 879 x 2372 47 and 37) and 1.4x (16-bit SYRK; past its
-# limits packed is up to 1.3x faster, 2230 x 89 13 us against 16). An
-# fp32 GEMM, whose kernels read any alignment, packs from F32_GEMM_PACK_FACTOR times that size: over random
-# unaligned shapes packing is 1.6x slower than in place at 2^30 multiply-adds,
+# times that size: over random shapes there they are 2.1x faster (batched bf16,
+# none slower, even from 2^30 on: 31 x (175 x 164 x 1098) 41 us packed, 20 in
+# place), 1.4x (fp32 SYRK, none slower; 879 x 2372 47 and 37) and about 2x
+# (16-bit SYRK, M-contiguous; 914 x 814 15.2 and 8.3). K-contiguous 16-bit SYRKs
+# are even (759 x 1139 16.2 and 15.5, 1267 x 411 12.4 and 14.0), and past the
+# limits of DIRECT_TILES packed is up to 1.3x faster (2230 x 89 13 and 16). An
+# fp32 GEMM, whose kernels read any alignment, packs from F32_GEMM_PACK_FACTOR
+# times that size: over random unaligned shapes packing is 1.6x slower than in place at 2^30 multiply-adds,
 # 1.26x at 2^33, 1.12x at 2^36, where cubes are even (4095^3 1100 us packed,
 # 1186 in place).
 PACK_MIN_MACS = {4: 1 << 30, 2: 1 << 28}
 F32_GEMM_PACK_FACTOR = 64
 # Largest numbers of 32 x 32 tiles (per launch, 256 CUs) of the unaligned 16-bit
-# GEMMs and the fp32 / 16-bit SYRKs that are packed only later, and the largest
-# k of those SYRKs
+# GEMMs and the fp32 / 16-bit SYRKs (these only M-contiguous) that are packed
+# only later, and the largest k of those SYRKs
 DIRECT_TILES = {"gemm": 12 * 256, "syrk": {4: (20 * 256, 4096), 2: (4 * 256, 2048)}}
 
 # TRNBLAS_GEMM_RAGGED=0 restores the reference's pad-first path
@@ -184,7 +186,7 @@ def _packed_syrk_operand(A, trans, a, t, lda, n, k):
     ev = 16 // A.element_size()
     least, tiles = _pack_min_macs(A.element_size(), True), -(-n // 32)
     most, longest = DIRECT_TILES["syrk"][A.element_size()]
-    if tiles * (tiles + 1) // 2 <= most and k <= longest:
+    if tiles * (tiles + 1) // 2 <= most and k <= longest and (ev == 4 or t):
         least *= 4
     if n * n * k < least or n == 0 or k == 0 or _dma_ready(a, lda, 0, n if t else k, ev):
         return a, t, lda, k
