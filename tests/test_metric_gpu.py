@@ -226,3 +226,15 @@ def test_metric_solve_host_route(dev, monkeypatch):
     monkeypatch.setenv("TRNBLAS_METRIC_SOLVE", "device")
     Xd = tb.metric_inv_half(J.to(dev))
     assert np.abs(Xd.cpu().numpy() - want).max() <= 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("at", [0, 1, 15, 16, 40, 130, 300])
+def test_metric_pivot_infinite(dev, at):
+    # an infinite pivot fails at its own column, whether or not columns follow it
+    from trnblas_amd.hip import kernels
+
+    for n in (at + 1, at + 3):
+        J = torch.eye(n, dtype=torch.float64, device=dev)
+        J[at, at] = float("inf")
+        _, info = kernels.metric_inv_half(J)
+        assert int(info) == at + 1

@@ -136,7 +136,7 @@ __device__ __forceinline__ double row_bcast(double v) {
 // One wave on a 16 x 16 diagonal sub-block `blk` (lower part read, SPD):
 // blk becomes L^-1 (blk = L L^T); in register e of lane (h = l / 16,
 // r = l % 16), l receives L[r][4 e + h] and y L^-1[4 e + h][r]. Returns 0, or
-// column + 1 of the first pivot that is not positive (or NaN) among the
+// column + 1 of the first pivot that is not positive and finite among the
 // leading nb columns.
 //
 // Elimination without square roots, U D U^T, four columns at a time: every
@@ -205,7 +205,7 @@ __device__ __forceinline__ int chol16(double* blk, double* ex, int lane, int nb,
   });
   // the lane that holds the pivot of column r
   const bool own = (r & 3) == h;
-  const unsigned long long b = __ballot(own && !(mine > 0.0) && r < nb);
+  const unsigned long long b = __ballot(own && !(mine > 0.0 && mine < __builtin_inf()) && r < nb);
   const unsigned cols = (unsigned)(b | b >> 16 | b >> 32 | b >> 48) & 0xffffu;
   if (own) ex[r] = rsqrt_nr(mine);
   __builtin_amdgcn_wave_barrier();
