@@ -501,6 +501,8 @@ int trnblas_hip_dgemm(int transA, int transB, int64_t M, int64_t N, int64_t K, d
  * and lower-triangle trailing updates, the trailing update on a second
  * stream of the same device so the next diagonal block runs beside it),
  * then L^-1 by recursive doubling over block halves and its transpose.
+ * With J[0] below 2^-960 the whole of J is factored as 2^120 times itself;
+ * else a pivot below 2^-1024 counts as not positive.
  * info (device int32) is set to the order of the first leading minor that
  * is not positive definite, else 0 (X is then garbage). workspace: at least
  * trnblas_hip_metric_inv_half_workspace(n) bytes, 256-byte aligned. Calls on

@@ -238,3 +238,30 @@ def test_metric_pivot_infinite(dev, at):
         J[at, at] = float("inf")
         _, info = kernels.metric_inv_half(J)
         assert int(info) == at + 1
+
+
+@pytest.mark.parametrize("n", [1, 3, 20, 150])
+@pytest.mark.parametrize("exp", [-1060, -1026, -1024, -1022, 1020])
+def test_metric_scale_at_the_ends_of_the_range(dev, n, exp):
+    # pivots below the normal range (or near its top): with J = 2^exp S for S of
+    # whole numbers, which a subnormal multiple represents exactly, X is 2^(-exp/2)
+    # times S's to rounding. Between 16-wide sub-blocks the update's 16 products and
+    # sums round to whole multiples of 2^-1074: 32 halves of one against pivots of
+    # 5 * 2^exp, halved in X (a root): below 2^(-1072 - exp).
+    from trnblas_amd.hip import kernels
+
+    v = torch.arange(n, dtype=torch.float64) % 3
+    S = torch.diag(torch.full((n,), 5.0, dtype=torch.float64)) + v[:, None] * v[None, :] * (0.0 if n > 20 else 1.0)
+    want, _ = kernels.metric_inv_half(S.to(dev))
+    J = torch.ldexp(S, torch.tensor(exp // 2)).ldexp(torch.tensor(exp - exp // 2))
+    X, info = kernels.metric_inv_half(J.to(dev))
+    assert int(info) == 0
+    got = torch.ldexp(X, torch.tensor(exp // 2, device=dev))
+    tol = 1e-14 + (2.0 ** (-1072 - exp) if exp < 0 else 0.0)
+    assert float((got - want).abs().max()) <= tol * float(want.abs().max())
+    if n <= kernels.CHOL_NB:  # the diagonal kernel by itself
+        Li, info = torch.empty_like(want), torch.zeros(1, dtype=torch.int32, device=dev)
+        kernels.chol_block(J.to(dev), Li, info, 0)
+        assert int(info) == 0
+        got = torch.ldexp(Li.mT, torch.tensor(exp // 2, device=dev))
+        assert float((got - want).abs().max()) <= tol * float(want.abs().max())

@@ -384,8 +384,13 @@ __device__ __forceinline__ void store_lower(const double* G, TT* Z, int64_t zr, 
 
 // LDS: the sub-block grid and a 16 x 16 scratch per wave, 96 KB, so the
 // workgroup shares a CU with a GEMM workgroup (64 KB) of a concurrent
-// stream instead of waiting for a whole free CU. zero_upper: the sub-blocks
+// stream instead of waiting for a whole free CU. chol16 divides by its
+// pivots, and 1 / d overflows below 2^-1024: with SCALE, a block with a diagonal
+// element below 2^-960 is factored as 2^120 times itself (a pivot that the
+// updates leave of a larger one is at least its rounding, 2^-53 of it; 1 us
+// more a block: the metric driver scales the whole matrix instead). zero_upper: the sub-blocks
 // of Li above its diagonal ones are cleared (else they hold zeros already).
+template <bool SCALE>
 __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, int64_t lda,
                                                            double* Li, int64_t ldl, int32_t* info,
                                                            int offset, int zero_upper) {
@@ -394,8 +399,16 @@ __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, in
   __shared__ double scr[NW][kSB];  // T of the inverse's block row; chol16's exchange
   const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // sub-block (i, k) of an accumulator to Z, rows and columns below nb
-  auto put = [&](double* Z, int64_t ld, int i, int k, const f64x4& v) __attribute__((always_inline)) {
+  bool small = false;
+  if constexpr (SCALE) {
+#pragma unroll
+    for (int x = lane; x < kCholNB; x += 64) small |= x < nb && A[(int64_t)x * (lda + 1)] < 0x1p-960;
+    small = __any(small);
+  }
+  // sub-block (i, k) of an accumulator to Z, rows and columns below nb; f: of a
+  // scaled block
+  auto put = [&](double* Z, int64_t ld, int i, int k, f64x4 v, double f) __attribute__((always_inline)) {
+    if (small) v *= f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int row = 16 * i + 4 * e + lg, col = 16 * k + li;
@@ -411,6 +424,7 @@ __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, in
       v[e] = row == col ? 1.0 : 0.0;
       if (row < nb && col <= row) v[e] = A[(int64_t)row * lda + col];
     }
+    if (small) v *= 0x1p120;
     return v;
   };
   int bad = 0;  // wave 0: the first pivot that is not positive, 1-based
@@ -445,6 +459,10 @@ __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, in
     // A. the panel (wave 0 has no row of it: it stores L_pp and its inverse)
     const int pi = p + NW - wave;
     if (wave == 0) {
+      if (small) {
+        l *= 0x1p-60;
+        y *= 0x1p60;
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int r = 16 * p + li, s = 16 * p + 4 * e + lg;
@@ -473,7 +491,7 @@ __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, in
       const int b = chol16(N, scr[0], lane, nb - 16 * (p + 1), l, y);
       if (bad == 0 && b != 0) bad = 16 * (p + 1) + b;
     } else {
-      if (pi < kNS) put(A, lda, pi, p, l);
+      if (pi < kNS) put(A, lda, pi, p, l, 0x1p-60);
       const int j = wave - 1;
       if (wave != 0 && j < p) {
         // t holds sum_{k < p - 1} L_pk Y_kj from the step before
@@ -482,7 +500,7 @@ __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, in
         __builtin_amdgcn_wave_barrier();
         y = f64x4{0.0, 0.0, 0.0, 0.0};
         mma16<false>(y, D, scr[wave], -1.0, lane);
-        put(Li, ldl, p, j, y);
+        put(Li, ldl, p, j, y, 0x1p60);
         t = f64x4{0.0, 0.0, 0.0, 0.0};
         if (!last)
           for (int k = j; k < p; ++k)
@@ -538,22 +556,24 @@ __global__ __launch_bounds__(kThreads) void trinv128_kernel(int n, int upper, in
 using namespace trnblas;
 
 int trnblas::chol_block(int64_t nb, double* A, int64_t lda, double* Linv, int64_t ldl,
-                        int32_t* info, int64_t offset, bool zero_upper, hipStream_t stream) {
+                        int32_t* info, int64_t offset, bool zero_upper, bool any_scale,
+                        hipStream_t stream) {
   TRNBLAS_CHECK_ARG(nb >= 0 && nb <= kCholNB, "chol_block: nb %lld not in [0, %d]", (long long)nb,
                     kCholNB);
   if (nb == 0) return TRNBLAS_OK;
   TRNBLAS_CHECK_ARG(A && Linv && info, "chol_block: NULL pointer");
   TRNBLAS_CHECK_ARG(lda >= nb && ldl >= nb, "chol_block: leading dimension below nb");
   TRNBLAS_CHECK_ARG(offset >= 0 && offset < (1ll << 30), "chol_block: bad offset");
-  hipLaunchKernelGGL(chol128_kernel, dim3(1), dim3(kThreads), 0, stream, (int)nb, A, lda, Linv, ldl,
-                     info, (int)offset, (int)zero_upper);
+  auto kern = any_scale ? chol128_kernel<true> : chol128_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3(1), dim3(kThreads), 0, stream, (int)nb, A, lda, Linv, ldl, info,
+                     (int)offset, (int)zero_upper);
   return check_launch("chol_block");
 }
 
 extern "C" int trnblas_hip_chol_block(int64_t nb, double* A, int64_t lda, double* Linv,
                                       int64_t ldl, int32_t* info, int64_t offset, void* stream) {
   clear_error();
-  return chol_block(nb, A, lda, Linv, ldl, info, offset, true, (hipStream_t)stream);
+  return chol_block(nb, A, lda, Linv, ldl, info, offset, true, true, (hipStream_t)stream);
 }
 
 extern "C" int trnblas_hip_tri_inv_blocks(int dtype, int64_t n, int upper, int unit, const void* T,

@@ -48,18 +48,20 @@ static dim3 grid2d(int64_t rows, int64_t cols) {
   return dim3((unsigned)(gx < 64 ? (gx > 0 ? gx : 1) : 64), (unsigned)(gy < 4096 ? (gy > 0 ? gy : 1) : 4096));
 }
 
-// X[j][i] = Y[i][j] for j <= i < n and zeros for j > i, through a 64 x 64 LDS
-// tile (both sides coalesced; only Y's lower tiles are read)
+// X[j][i] = f Y[i][j] for j <= i < n and zeros for j > i, through a 64 x 64 LDS
+// tile (both sides coalesced; only Y's lower tiles are read); f: metric_init_kernel's
 __global__ __launch_bounds__(256) void transpose_kernel(int n, const double* Y, int64_t ldy,
-                                                        double* X, int64_t ldx) {
+                                                        const double* factor, double* X,
+                                                        int64_t ldx) {
   __shared__ double t[64][65];
+  const double f = *factor;
   const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   if (i0 >= j0) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int i = i0 + ty + 4 * r, j = j0 + tx;
-      t[ty + 4 * r][tx] = i < n && j <= i ? Y[(int64_t)i * ldy + j] : 0.0;
+      t[ty + 4 * r][tx] = i < n && j <= i ? f * Y[(int64_t)i * ldy + j] : 0.0;
     }
     __syncthreads();
   }
@@ -72,19 +74,26 @@ __global__ __launch_bounds__(256) void transpose_kernel(int n, const double* Y, 
 
 // W's lower 128 x 128 blocks = J's, zeros past n; zeros in Y's last diagonal
 // block when it is partial (its padding takes part in the products); info =
-// 0. Grid: (blocks of a row, block rows, 8 slices of 16 rows).
+// 0. A metric whose first diagonal element is below 2^-960 is factored as 2^120
+// times itself (the diagonal kernel divides by the pivots, and 1 / d overflows
+// below 2^-1024), and *factor brings X back. Grid: (blocks of a row, block rows, 8 slices of 16 rows).
 __global__ __launch_bounds__(256) void metric_init_kernel(int64_t n, int64_t npad, const double* J,
                                                           int64_t ldj, double* W, double* Y,
-                                                          int32_t* info) {
+                                                          double* factor, int32_t* info) {
   const int64_t bi = blockIdx.y, bj = blockIdx.x;
   if (bj > bi) return;
-  if (bi == 0 && blockIdx.z == 0 && threadIdx.x == 0) *info = 0;
+  const bool small = J[0] < 0x1p-960;
+  if (bi == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
+    *factor = small ? 0x1p60 : 1.0;
+    *info = 0;
+  }
   const bool tail = bi == bj && (bi + 1) * 128 > n;
+  const double f = small ? 0x1p120 : 1.0;
   const int64_t j = bj * 128 + (threadIdx.x & 127);
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
     const int64_t i = bi * 128 + blockIdx.z * 16 + (threadIdx.x >> 7) + 2 * u;
-    W[i * npad + j] = i < n && j < n ? J[i * ldj + j] : 0.0;
+    W[i * npad + j] = i < n && j < n ? f * J[i * ldj + j] : 0.0;
     if (tail) Y[i * npad + j] = 0.0;
   }
 }
@@ -129,7 +138,7 @@ static int side_init(SideStream* ss) {
   return TRNBLAS_OK;
 }
 
-static void metric_layout(int64_t n, int64_t& npad, size_t off[5]) {
+static void metric_layout(int64_t n, int64_t& npad, size_t off[6]) {
   npad = (n + kNB - 1) / kNB * kNB;
   const size_t sq = (size_t)npad * npad * 8;
   auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -138,6 +147,7 @@ static void metric_layout(int64_t n, int64_t& npad, size_t off[5]) {
   off[2] = up(off[1] + sq);                  // Y: L^-1 (diagonal blocks from the kernel)
   off[3] = up(off[2] + sq);                  // T: a step's rows L[B, :k0] Y[:k0, :k0]
   off[4] = up(off[3] + (size_t)kStep * npad * 8);  // S: L_10 Y_00 of a step's blocks 0, 1
+  off[5] = up(off[4] + (size_t)kNB * kNB * 8);     // the factor of X
 }
 
 #define TRY(x)                        \
@@ -153,9 +163,9 @@ using namespace trnblas;
 extern "C" size_t trnblas_hip_metric_inv_half_workspace(int64_t n) {
   if (n <= 0) return 0;
   int64_t npad;
-  size_t off[5];
+  size_t off[6];
   metric_layout(n, npad, off);
-  return off[4] + (size_t)kNB * kNB * 8;
+  return off[5] + sizeof(double);
 }
 
 extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t ldj, double* X,
@@ -173,7 +183,7 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
                     "metric_inv_half: workspace must be 256-byte aligned");
   hipStream_t main = (hipStream_t)stream;
   int64_t npad;
-  size_t off[5];
+  size_t off[6];
   metric_layout(n, npad, off);
   char* ws = static_cast<char*>(workspace);
   double* W = reinterpret_cast<double*>(ws + off[0]);
@@ -181,6 +191,7 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
   double* Y = reinterpret_cast<double*>(ws + off[2]);
   double* T = reinterpret_cast<double*>(ws + off[3]);
   double* S = reinterpret_cast<double*>(ws + off[4]);
+  double* factor = reinterpret_cast<double*>(ws + off[5]);
   int rc = TRNBLAS_OK;
   SideStream* ss = side_stream(rc);
   if (!ss) return rc;
@@ -195,7 +206,7 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
 
   const unsigned nblk = (unsigned)(npad / kNB);
   hipLaunchKernelGGL(metric_init_kernel, dim3(nblk, nblk, 8), dim3(256), 0, main, n, npad, J, ldj, W,
-                     Y, info);
+                     Y, factor, info);
   TRY(check_launch("metric_inv_half(init)"));
   // D = alpha A op(B) + beta D over blocks of W, L, Y (ld npad)
   auto mm = [&](bool bt, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
@@ -206,7 +217,7 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
   };
   auto chol = [&](int64_t k) {  // L_bb into W (lower triangle), L_bb^-1 = Y_bb into Y
     return chol_block(n - k < kNB ? n - k : kNB, W + k * npad + k, npad, Y + k * npad + k, npad, info,
-                      k, true, main);
+                      k, true, false, main);
   };
 
   // up to two steps there is no trailing update, and the hand-overs to the
@@ -267,7 +278,8 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
     TRY(wait(main, ss->inverted));
   }
   const unsigned tb = (unsigned)((n + 63) / 64);
-  hipLaunchKernelGGL(transpose_kernel, dim3(tb, tb), dim3(256), 0, main, (int)n, Y, npad, X, ldx);
+  hipLaunchKernelGGL(transpose_kernel, dim3(tb, tb), dim3(256), 0, main, (int)n, Y, npad,
+                     factor, X, ldx);
   return check_launch("metric_inv_half(transpose)");
 }
 
