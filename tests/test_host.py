@@ -618,3 +618,35 @@ def test_unaligned_syrk_packing_starts_later_on_small_grids(monkeypatch, dtype, 
     A = torch.zeros(1, dtype=dtype).expand(*((kk, n) if trans else (n, kk)))
     k._packed_syrk_operand(A, trans, A, trans, A.shape[1], n, kk)
     assert bool(seen) == packs
+
+
+@pytest.mark.parametrize("dtype,shape,ta,tb,lda,ldb", [
+    (torch.float32, (40, 16_800_001, 100), False, False, 100, 16_800_001),  # B N-contiguous, 2^24 and more apart
+    (torch.float32, (601, 602, 3001), False, False, 4_300_001, 602),  # A K-contiguous, 2^22 and more apart
+    (torch.bfloat16, (512, 513, 2048), True, True, 16_800_001, 2048),
+])  # fmt: skip
+def test_operands_past_32_bit_panel_offsets_are_packed(monkeypatch, dtype, shape, ta, tb, lda, ldb):
+    # the launcher refuses such leading dimensions in place, so they are packed
+    # from PACK_MIN_MACS on also where smaller ones are read in place
+    from trnblas_amd.hip import kernels as k
+
+    seen = []
+    monkeypatch.setattr(k, "_pack_k", lambda X, kp: seen.append(kp) or X)
+    M, N, K = shape
+    A, B = torch.zeros(1, dtype=dtype).expand(M, K), torch.zeros(1, dtype=dtype).expand(K, N)
+    k._packed_operands(A, B, A, ta, M if ta else K, 0, B, tb, K if tb else 602, 0, M, N, K, 1)
+    assert not seen
+    k._packed_operands(A, B, A, ta, lda, 0, B, tb, ldb, 0, M, N, K, 1)
+    assert seen
+
+
+def test_syrk_operand_past_32_bit_panel_offsets_is_packed(monkeypatch):
+    from trnblas_amd.hip import kernels as k
+
+    seen = []
+    monkeypatch.setattr(k, "_pack_k", lambda X, kp: seen.append(kp) or X)
+    A = torch.zeros(1).expand(4001, 533)
+    k._packed_syrk_operand(A, True, A, True, 533, 533, 4001)
+    assert not seen
+    k._packed_syrk_operand(A, True, A, True, 16_800_001, 533, 4001)
+    assert seen

@@ -137,6 +137,12 @@ def _pack_min_macs(elem_size: int, syrk: bool = False) -> int:
     return PACK_MIN_MACS[elem_size] * (F32_GEMM_PACK_FACTOR if elem_size == 4 and not syrk else 1)
 
 
+def _panel_fits(k_contiguous: bool, ld: int, elem_size: int) -> bool:
+    """Whether the launcher's 32-bit offsets reach over one panel of an operand
+    with this leading dimension; it refuses larger ones, which serve only packed."""
+    return (128 if k_contiguous else 128 // elem_size) * ld * elem_size < 0x7FFFFFF0 - 64
+
+
 def _dma_ready(t: torch.Tensor, ld: int, stride: int, ext: int, ev: int) -> bool:
     return t.data_ptr() % 16 == 0 and ld % ev == 0 and stride % ev == 0 and ext % ev == 0
 
@@ -164,6 +170,8 @@ def _packed_operands(A, B, a, ta, lda, sa, b, tb, ldb, sb, M, N, K, nb):
     least = _pack_min_macs(A.element_size())
     if ev == 8 and nb * -(-M // 32) * -(-N // 32) <= DIRECT_TILES["gemm"]:
         least *= 4
+    if not (_panel_fits(not ta, lda, A.element_size()) and _panel_fits(tb, ldb, A.element_size())):
+        least = min(least, PACK_MIN_MACS[A.element_size()])
     if nb * M * N * K < least or M == 0 or N == 0 or K == 0:
         return a, ta, lda, sa, b, tb, ldb, sb, K
     a_ok = _dma_ready(a, lda, sa, M if ta else K, ev)
@@ -188,6 +196,8 @@ def _packed_syrk_operand(A, trans, a, t, lda, n, k):
     most, longest = DIRECT_TILES["syrk"][A.element_size()]
     if tiles * (tiles + 1) // 2 <= most and k <= longest and (ev == 4 or t):
         least *= 4
+    if not _panel_fits(not t, lda, A.element_size()):
+        least = min(least, PACK_MIN_MACS[A.element_size()])
     if n * n * k < least or n == 0 or k == 0 or _dma_ready(a, lda, 0, n if t else k, ev):
         return a, t, lda, k
     kp = -(-k // ev) * ev
