@@ -95,6 +95,17 @@ int trnblas_hip_gemm(int dtype, int transA, int transB, int64_t M, int64_t N, in
 size_t trnblas_hip_gemm_workspace(void);
 
 /*
+ * The name of the kernel that trnblas_hip_gemm (trnblas_hip_syrk for syrk !=
+ * 0: M == N, transA its trans, transB and ldb unused) launches for a product
+ * with these sizes, 16-byte aligned operands of the given leading dimensions
+ * (batches back to back) and the full workspace, or NULL with the last error
+ * set when it refuses them. Launches nothing and needs no GPU (256 CUs are
+ * assumed without one).
+ */
+const char* trnblas_hip_gemm_plan(int dtype, int syrk, int transA, int transB, int64_t M,
+                                  int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t batch);
+
+/*
  * Operand packing:  P[b] (R x kp, row-major) = X[b] (R x K) with zero
  * columns K .. kp - 1.
  *

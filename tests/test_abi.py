@@ -98,3 +98,49 @@ def test_syrk_and_triangle_argument_errors_without_a_gpu():
     assert rc == _lib.E_ARG and b"aligned" in lib.trnblas_hip_last_error()
     rc = lib.trnblas_hip_chol_block(129, fake, 129, fake, 129, fake, 0, None)
     assert rc == _lib.E_ARG and b"nb" in lib.trnblas_hip_last_error()
+
+
+def _plan(dtype, syrk, ta, tb, M, N, K, batch=1):
+    from trnblas_amd.hip import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("library not built")
+    name = _lib.load().trnblas_hip_gemm_plan(dtype, syrk, ta, tb, M, N, K, M if ta else K, K if tb else N, batch)
+    assert name is not None, _lib.load().trnblas_hip_last_error()
+    return name.decode()
+
+
+F32, BF16, F16 = 0, 1, 2
+
+
+@pytest.mark.parametrize("ta", [0, 1])
+@pytest.mark.parametrize("tb", [0, 1])
+@pytest.mark.parametrize("M,N,K,batch,direct", [
+    (64, 64, 2048, 1, True), (64, 64, 65536, 1, False), (128, 128, 32768, 1, False), (256, 256, 16384, 1, False),
+    (8, 32, 276928, 4, False), (63, 61, 2047, 1, True), (63, 61, 65537, 1, False), (3, 20, 110293, 1, False),
+    (1, 1, 1 << 22, 1, False),
+])  # fmt: skip
+def test_16bit_gemm_of_few_tiles_and_long_k_is_split(M, N, K, batch, direct, ta, tb):
+    # hgemm_direct_kernel runs a tile's whole K in one workgroup: products of few
+    # tiles and long K belong on the stream-K kernels
+    for dtype in (BF16, F16):
+        assert (_plan(dtype, 0, ta, tb, M, N, K, batch) == "hgemm_direct_kernel") == direct
+
+
+@pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("n,k,direct", [(64, 2048, True), (64, 8192, False), (56, 181568, False), (59, 2047, True),
+                                        (59, 132806, False), (13, 74125, False)])  # fmt: skip
+def test_16bit_syrk_of_few_tiles_and_long_k_is_split(n, k, direct, trans):
+    assert (_plan(BF16, 1, trans, 0, n, n, k) == "hgemm_direct_kernel") == direct
+
+
+def test_gemm_plan_refuses_what_the_launch_refuses():
+    from trnblas_amd.hip import _lib
+
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("library not built")
+    lib = _lib.load()
+    assert lib.trnblas_hip_gemm_plan(0, 0, 0, 0, 4, 1 << 24, 4, 4, 1 << 24, 1) is None
+    assert b"32-bit panel offsets" in lib.trnblas_hip_last_error()
+    assert lib.trnblas_hip_gemm_plan(7, 0, 0, 0, 4, 4, 4, 4, 4, 1) is None
+    assert lib.trnblas_hip_gemm_plan(0, 1, 0, 0, 4, 5, 4, 4, 5, 1) is None

@@ -590,6 +590,7 @@ def test_ozaki_plan_known_answers():
     (torch.bfloat16, (1023, 1023, 1023), False), (torch.bfloat16, (1025, 1025, 1025), True),  # 2^30, few tiles
     (torch.bfloat16, (3201, 1025, 99), True),  # more than 12 tiles per CU, 2^28
     (torch.float32, (1023, 1023, 1027), False),
+    (torch.bfloat16, (86, 29, 168729), True),  # few tiles and long K
 ])  # fmt: skip
 def test_unaligned_gemm_packing_starts_later_on_small_grids(monkeypatch, dtype, shape, packs):
     # sizes only: the operands are expanded scalars, and packing is recorded

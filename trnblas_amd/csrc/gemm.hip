@@ -1411,6 +1411,7 @@ static int launch_narrow(GemmArgs g, size_t ws_bytes, hipStream_t s) {
   // unused dynamic LDS caps it at two (64 KiB each)
   g.sk_groups = choose_sk(g, 2, ws_bytes);  // (its slot check assumes 64 KiB partials: 32 here)
   const int grid = g.sk_groups ? g.sk_groups : g.ntiles;
+  if (planned(g, "gemm_dma_kernel narrow")) return TRNBLAS_OK;
   hipLaunchKernelGGL((gemm_dma_kernel<T, AKC, BKC, false, 64>), dim3(grid), dim3(256),
                      kNarrowLdsPad, s, g);
   int rc = check_launch("trnblas_hip_gemm");
@@ -1427,6 +1428,7 @@ static int launch_pipe(GemmArgs g, hipStream_t s) {
   g.span = chain_length(g.K, 4) / kPipeBK;
   g.vec2 = g.ldd % 2 == 0 && (reinterpret_cast<uintptr_t>(g.D) & 7) == 0 &&
            (g.C == nullptr || (g.ldc % 2 == 0 && (reinterpret_cast<uintptr_t>(g.C) & 7) == 0));
+  if (planned(g, "sgemm_pipe_kernel")) return TRNBLAS_OK;
   hipLaunchKernelGGL(sgemm_pipe_kernel, dim3(g.ntiles), dim3(kPipeThreads), 0, s, g);
   return check_launch("trnblas_hip_gemm");
 }
@@ -1469,6 +1471,7 @@ static int launch_wide(GemmArgs g, hipStream_t s) {
   g.tiles_n = (g.N + 255) / 256;
   g.ntiles = g.tiles_m * g.tiles_n * g.batch;
   g.nk = (g.K + 63) / 64;
+  if (planned(g, "hgemm256_kernel")) return TRNBLAS_OK;
   hipLaunchKernelGGL((hgemm256_kernel<T, AKC, BKC>), dim3(g.ntiles), dim3(512), 0, s, g);
   return check_launch("trnblas_hip_gemm");
 }
@@ -1491,6 +1494,7 @@ static bool one_round_pays(const GemmArgs& g) {
 
 template <typename T, bool AKC, bool BKC>
 static int launch_one_round(const GemmArgs& g, hipStream_t s) {
+  if (planned(g, "hgemm128_kernel")) return TRNBLAS_OK;
   hipLaunchKernelGGL((hgemm128_kernel<T, AKC, BKC>), dim3(g.ntiles), dim3(64 * (kHCompute + 4)), 0, s,
                      g);
   return check_launch("trnblas_hip_gemm");
@@ -1515,6 +1519,7 @@ static int launch_t(GemmArgs g, size_t ws_bytes, hipStream_t s) {
   if constexpr (DMA && !SYRK) {
     if (narrow_tiles_pay(g, (int)sizeof(T))) return launch_narrow<T, AKC, BKC>(g, ws_bytes, s);
   }
+  if (planned(g, DMA ? "gemm_dma_kernel" : "gemm_kernel")) return TRNBLAS_OK;
   void (*kern)(GemmArgs);
   if constexpr (DMA)
     kern = gemm_dma_kernel<T, AKC, BKC, SYRK>;
@@ -1808,6 +1813,46 @@ extern "C" int trnblas_hip_syrk_flagged(int dtype, int uplo, int trans, int64_t 
   TRNBLAS_CHECK_ARG(flags != nullptr || beta == 0.0, "syrk_flagged: NULL flags");
   return syrk_impl(dtype, uplo, trans, N, K, alpha, A, lda, beta, C, ldc, D, ldd, flags,
                    workspace, workspace_bytes, stream);
+}
+
+extern "C" const char* trnblas_hip_gemm_plan(int dtype, int syrk, int transA, int transB, int64_t M,
+                                             int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                             int64_t batch) {
+  clear_error();
+  const bool half = dtype == TRNBLAS_BF16 || dtype == TRNBLAS_F16;
+  if ((dtype != TRNBLAS_F32 && !half) || M < 1 || N < 1 || K < 1 || batch < 1 || M >= (1ll << 31) ||
+      N >= (1ll << 31) || K >= (1ll << 31) || (syrk && (M != N || batch != 1))) {
+    set_error("gemm_plan: bad arguments");
+    return nullptr;
+  }
+  const char* name = nullptr;
+  GemmArgs g{};
+  g.plan = &name;
+  g.M = (int)M;
+  g.N = (int)N;
+  g.K = (int)K;
+  g.alpha = 1.0f;
+  // (16-byte aligned bases and a workspace, which nothing reads)
+  g.A = g.B = reinterpret_cast<const void*>(4096);
+  g.ws = reinterpret_cast<float*>(4096);
+  g.lda = lda;
+  g.ldb = syrk ? lda : ldb;
+  g.sA = batch > 1 ? lda * (transA ? K : M) : 0;
+  g.sB = batch > 1 ? ldb * (transB ? N : K) : 0;
+  g.ldd = N;
+  g.batch = (int)batch;
+  g.tiles_m = (int)((M + kTileM - 1) / kTileM);
+  g.tiles_n = (int)((N + kTileN - 1) / kTileN);
+  const int64_t t = g.tiles_m, ntiles = syrk ? t * (t + 1) / 2 : t * g.tiles_n * batch;
+  if (ntiles >= (1ll << 31)) {
+    set_error("gemm_plan: too many tiles");
+    return nullptr;
+  }
+  g.ntiles = (int)ntiles;
+  g.nk = (int)((K + k_tile(dtype) - 1) / k_tile(dtype));
+  const int rc = syrk ? dispatch<true>(dtype, g, !transA, !transA, trnblas_hip_gemm_workspace(), nullptr)
+                      : dispatch<false>(dtype, g, !transA, transB != 0, trnblas_hip_gemm_workspace(), nullptr);
+  return rc ? nullptr : name;
 }
 
 // Which strict triangles of an n x n matrix hold a nonzero (NaN counts), for

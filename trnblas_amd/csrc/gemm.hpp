@@ -31,7 +31,14 @@ struct GemmArgs {
   float* ws;             // stream-K partial tiles [sk_groups][2][BM * BN]
   int span;              // k-tiles per MFMA accumulation chain (chain_length / k-tile)
   int splits;            // sgemm.hip: k ranges per tile, partial tiles in ws (1 = whole tiles)
+  const char** plan;     // trnblas_hip_gemm_plan: receives the kernel's name, nothing is launched
 };
+
+// True when only the kernel's name is asked for.
+static inline bool planned(const GemmArgs& g, const char* kernel) {
+  if (g.plan) *g.plan = kernel;
+  return g.plan != nullptr;
+}
 
 // Accumulation: the MFMA accumulator of a tile restarts from zero every
 // chain_length(K) k values and each finished chain is added into a separate

@@ -243,6 +243,7 @@ static int run_direct(int waves, GemmArgs g, hipStream_t s) {
   g.tiles_n = (g.N + 31) / 32;
   g.ntiles = SYRK ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * g.tiles_n * g.batch;
   g.span = chain_length(g.K, 2) / 32;
+  if (planned(g, "hgemm_direct_kernel")) return TRNBLAS_OK;
   if (waves == 4)
     hipLaunchKernelGGL((hgemm_direct_kernel<T, 4, AKC, BKC, ODD, SYRK>), dim3(g.ntiles), dim3(256), 0, s, g);
   else
@@ -253,10 +254,15 @@ static int run_direct(int waves, GemmArgs g, hipStream_t s) {
 // Where it serves (q: 32 x 32 tiles per CU, ch: 32-wide chunks of K): products
 // of up to a few tiles per CU, whose time is launch, latency and, on the
 // 128 x 128 kernels, instruction fetch and idle CUs. Aligned operands: q <= 6
-// (SYRK 12) and q ch <= 200; above, the LDS-DMA kernels read each operand less
+// (SYRK 8) and q ch <= 200; above, the LDS-DMA kernels read each operand less
 // often from L2. Unaligned ones up to q = 12 (SYRK 20): gemm_kernel runs
 // them at half this kernel's rate, but for K of a few values, where the store
-// of D counts and larger tiles store longer rows.
+// of D counts and larger tiles store longer rows. The limits of ch are where
+// one workgroup's serial chain takes as long as stream-K over the chip: 64 x
+// 64 x 65536 (4 workgroups) 130 us here and 27 there, SYRK 56 x 181568 609 and
+// 47. Both operands K-contiguous read 32 rows at once, words of odd rows five
+// at a time, so these limits are lower (aligned 80 x 4416 SYRK 17.8 us here, 12.6
+// there; unaligned 58 x 7427 37.8 and 27.4).
 // Over 707 random GEMMs and 64 SYRKs (bf16, fp16; M, N, K 1 .. 4096, batches
 // to 64) against gemm.hip's kernels: aligned 1.70x and 2.0x faster on average,
 // unaligned 2.85x and 2.7x, none slower. GPU time (us) before / after, the
@@ -268,14 +274,17 @@ template <typename T, bool SYRK>
 bool hgemm_launch(const GemmArgs& g, bool akc, bool bkc, bool aligned, hipStream_t s, int* rc) {
   const double tm = (g.M + 31) / 32, tn = (g.N + 31) / 32, ch = (g.K + 31) / 32;
   const double q = (SYRK ? 0.5 * tm * (tm + 1.0) : tm * tn * g.batch) / device_cus();
-  if (aligned ? q > (SYRK ? 12.0 : 6.0) || q * ch > 200.0 : q > (SYRK ? 20.0 : 12.0)) return false;
-  const double t4 = 3.3 + std::max(0.31 * std::ceil(ch / 4), 0.096 * q * ch) + 0.45 * q;
-  const double t8 = 3.0 + std::max(0.58 * std::ceil(ch / 8), 0.092 * q * ch) + 0.88 * q;
-  const int waves = t4 <= t8 ? 4 : 8;
   auto odd = [](const void* p, int64_t ld, int64_t st) {
     return (((uintptr_t)p >> 1 | ld | st) & 1) != 0;
   };
   const bool words = (akc && odd(g.A, g.lda, g.sA)) || (bkc && odd(g.B, g.ldb, g.sB));
+  const bool kk = akc && bkc;
+  if (aligned ? q > (kk ? 5.0 : SYRK ? 8.0 : 6.0) || ch > (kk ? 96.0 : 192.0) || q * ch > (kk ? 120.0 : 200.0)
+              : q > (SYRK ? 20.0 : 12.0) || ch > (words ? (kk ? 128.0 : 256.0) : SYRK ? 256.0 : 384.0))
+    return false;
+  const double t4 = 3.3 + std::max(0.31 * std::ceil(ch / 4), 0.096 * q * ch) + 0.45 * q;
+  const double t8 = 3.0 + std::max(0.58 * std::ceil(ch / 8), 0.092 * q * ch) + 0.88 * q;
+  const int waves = t4 <= t8 ? 4 : 8;
   if constexpr (SYRK) {
     *rc = !akc    ? run_direct<T, false, false, false, true>(waves, g, s)
           : words ? run_direct<T, true, true, true, true>(waves, g, s)

@@ -475,6 +475,7 @@ static int run_tile(GemmArgs g, int splits, size_t ws_bytes, hipStream_t s) {
   g.splits = splits;
   if (splits > 1 && (g.ws == nullptr || (size_t)g.ntiles * splits * BM * BN * 4 > ws_bytes))
     g.splits = 1;
+  if (planned(g, g.splits > 1 ? "sgemm_tile_kernel split" : "sgemm_tile_kernel")) return TRNBLAS_OK;
   hipLaunchKernelGGL((sgemm_tile_kernel<BM, BN, WGM, AKC, BKC>), dim3(g.ntiles * g.splits), dim3(256), 0,
                      s, g);
   int rc = check_launch("trnblas_hip_gemm");
@@ -489,6 +490,7 @@ static int run_direct(GemmArgs g, hipStream_t s) {
   g.tiles_n = (g.N + 31) / 32;
   g.ntiles = SYRK ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * g.tiles_n * g.batch;
   g.span = chain_length(g.K, 4) / 16;
+  if (planned(g, "sgemm_direct_kernel")) return TRNBLAS_OK;
   hipLaunchKernelGGL((sgemm_direct_kernel<WAVES, AKC, BKC, SYRK>), dim3(g.ntiles), dim3(64 * WAVES), 0,
                      s, g);
   return check_launch(SYRK ? "trnblas_hip_syrk" : "trnblas_hip_gemm");

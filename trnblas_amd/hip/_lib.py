@@ -47,6 +47,10 @@ SIGNATURES = {
         + [_c_ptr],
     ),
     "trnblas_hip_gemm_workspace": (_c_size, []),
+    "trnblas_hip_gemm_plan": (
+        ctypes.c_char_p,
+        [_c_int, _c_int, _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64],
+    ),
     "trnblas_hip_pack_k": (
         _c_int,
         [_c_int, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64]
