@@ -144,3 +144,11 @@ def test_gemm_plan_refuses_what_the_launch_refuses():
     assert b"32-bit panel offsets" in lib.trnblas_hip_last_error()
     assert lib.trnblas_hip_gemm_plan(7, 0, 0, 0, 4, 4, 4, 4, 4, 1) is None
     assert lib.trnblas_hip_gemm_plan(0, 1, 0, 0, 4, 5, 4, 4, 5, 1) is None
+
+
+def test_16bit_one_round_kernel_counts_half_tiles():
+    # gemm_dma_kernel's 128 x 64 tiles do half the work where N is at most 64: with
+    # many k-tiles they are faster than hgemm128_kernel's whole 128 x 128 ones
+    for M, N, K, b in ((408, 8, 10264, 37), (1168, 24, 6592, 17)):
+        assert _plan(BF16, 0, 1, 0, M, N, K, b) == "gemm_dma_kernel narrow"
+    assert _plan(BF16, 0, 0, 0, 1784, 2032, 2048) == "hgemm128_kernel"

@@ -1479,7 +1479,8 @@ static int launch_wide(GemmArgs g, hipStream_t s) {
 // hgemm128_kernel for up to one 128 x 128 tile per CU, unless enough k-tiles
 // let gemm_dma_kernel's narrow tiles / stream-K split them better: few tiles,
 // by the two kernels' times (about 6 + 0.62 nk us against 12 + 0.004 nk tiles
-// from 20 k-tiles on), or a round that narrow tiles fill as well. Measured
+// from 20 k-tiles on, tiles counted in halves of 64 columns: 37 x (408 x 8 x
+// 10264) 118 / 81), or a round that narrow tiles fill as well. Measured
 // (bf16, us, NN, against gemm_dma_kernel): 504 x 496 x 512 10.4 / 11.9, 1016 x
 // 1008 x 1024 15.6 / 20.5, 1784 x 2032 x 2048 28.5 / 60.5, 2048^2 x 1024 18.3 /
 // 29.9, 64 x (256^2 x 1024) 19.7 / 30.5; left to it: 504 x 496 x 2048 (24.1) /
@@ -1488,7 +1489,8 @@ static bool one_round_pays(const GemmArgs& g) {
   const double t = g.ntiles, cus = device_cus(), nk = g.nk;
   if (t > cus) return false;
   if (t < cus / 8) return nk < 16;
-  if (nk >= 20 && nk * (0.62 - 1.024 * t / cus) > 6.0) return false;
+  const double work = 0.5 * (double)g.tiles_m * (double)((g.N + 63) / 64) * (double)g.batch;
+  if (nk >= 20 && nk * (0.62 - 1.024 * work / cus) > 6.0) return false;
   return t < 0.9 * cus || nk < 24;
 }
 
