@@ -152,3 +152,8 @@ def test_16bit_one_round_kernel_counts_half_tiles():
     for M, N, K, b in ((408, 8, 10264, 37), (1168, 24, 6592, 17)):
         assert _plan(BF16, 0, 1, 0, M, N, K, b) == "gemm_dma_kernel narrow"
     assert _plan(BF16, 0, 0, 0, 1784, 2032, 2048) == "hgemm128_kernel"
+
+
+@pytest.mark.parametrize("M,N,K,batch", [(1200, 256, 4792, 1), (816, 368, 4344, 1), (40, 232, 5544, 18)])
+def test_16bit_gemm_of_a_tile_per_cu_and_long_k(M, N, K, batch):
+    assert _plan(BF16, 0, 1, 0, M, N, K, batch) != "hgemm_direct_kernel"

@@ -254,7 +254,8 @@ static int run_direct(int waves, GemmArgs g, hipStream_t s) {
 // Where it serves (q: 32 x 32 tiles per CU, ch: 32-wide chunks of K): products
 // of up to a few tiles per CU, whose time is launch, latency and, on the
 // 128 x 128 kernels, instruction fetch and idle CUs. Aligned operands: q <= 6
-// (SYRK 8) and q ch <= 200; above, the LDS-DMA kernels read each operand less
+// (SYRK 8) and q ch <= 200 (150 past 96 chunks: 1200 x 256 x 4792, 178, 30.3 us
+// here, 23.8 on narrow tiles); above, the LDS-DMA kernels read each operand less
 // often from L2. Unaligned ones up to q = 12 (SYRK 20): gemm_kernel runs
 // them at half this kernel's rate, but for K of a few values, where the store
 // of D counts and larger tiles store longer rows. The limits of ch are where
@@ -279,7 +280,8 @@ bool hgemm_launch(const GemmArgs& g, bool akc, bool bkc, bool aligned, hipStream
   };
   const bool words = (akc && odd(g.A, g.lda, g.sA)) || (bkc && odd(g.B, g.ldb, g.sB));
   const bool kk = akc && bkc;
-  if (aligned ? q > (kk ? 5.0 : SYRK ? 8.0 : 6.0) || ch > (kk ? 96.0 : 192.0) || q * ch > (kk ? 120.0 : 200.0)
+  if (aligned ? q > (kk ? 5.0 : SYRK ? 8.0 : 6.0) || ch > (kk ? 96.0 : 192.0) ||
+                    q * ch > (kk ? 120.0 : ch > 96.0 ? 150.0 : 200.0)
               : q > (SYRK ? 20.0 : 12.0) || ch > (words ? (kk ? 128.0 : 256.0) : SYRK ? 256.0 : 384.0))
     return false;
   const double t4 = 3.3 + std::max(0.31 * std::ceil(ch / 4), 0.096 * q * ch) + 0.45 * q;
