@@ -99,7 +99,8 @@ size_t trnblas_hip_gemm_workspace(void);
  * 0: M == N, transA its trans, transB and ldb unused) launches for a product
  * with these sizes, 16-byte aligned operands of the given leading dimensions
  * (batches back to back) and the full workspace, or NULL with the last error
- * set when it refuses them. Launches nothing and needs no GPU (256 CUs are
+ * set when it refuses them ("in S": K split over S workgroups a tile; valid
+ * until the thread's next call). Launches nothing and needs no GPU (256 CUs are
  * assumed without one).
  */
 const char* trnblas_hip_gemm_plan(int dtype, int syrk, int transA, int transB, int64_t M,

@@ -157,3 +157,14 @@ def test_16bit_one_round_kernel_counts_half_tiles():
 @pytest.mark.parametrize("M,N,K,batch", [(1200, 256, 4792, 1), (816, 368, 4344, 1), (40, 232, 5544, 18)])
 def test_16bit_gemm_of_a_tile_per_cu_and_long_k(M, N, K, batch):
     assert _plan(BF16, 0, 1, 0, M, N, K, batch) != "hgemm_direct_kernel"
+
+
+def test_fp32_gemm_of_few_tiles_and_long_k_is_split():
+    # unaligned products have no stream-K kernel: K goes over as many workgroups as
+    # the chip holds, and no workgroup walks tens of thousands of k alone
+    for K, least in ((65537, 64), (300001, 128), (1000001, 256)):
+        name = _plan(F32, 0, 0, 0, 63, 63, K)
+        assert name.startswith("sgemm_tile_kernel<64, 64> in") and int(name.split()[-1]) >= least, name
+    assert "direct" not in _plan(F32, 0, 0, 0, 549, 174, 41161, 10)
+    # aligned, N <= 64: narrow tiles are half the work
+    assert _plan(F32, 0, 0, 1, 66, 3, 33628, 10) == "gemm_dma_kernel narrow"

@@ -633,6 +633,33 @@ def test_sgemm_any_alignment(dev, M, N, K, batch, ta, tb):
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("M,N,K,batch", [(63, 61, 65537, 1), (1, 1, 300001, 1), (5, 130, 70001, 2), (129, 65, 66003, 1)])
+def test_sgemm_many_splits(dev, M, N, K, batch, ta, tb):
+    # few tiles and a long K, split over up to 512 workgroups a tile whose sums one
+    # kernel adds: the same bits twice, and fp64 at the fp32 gate
+    from trnblas_amd.hip import kernels
+
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 7 * K)
+    A = torch.randn(batch, *((K, M) if ta else (M, K)), generator=g, device=dev)
+    B = torch.randn(batch, *((N, K) if tb else (K, N)), generator=g, device=dev)
+    A, B = (A.mT if ta else A), (B.mT if tb else B)
+    C = torch.randn(batch, M, N, generator=g, device=dev)
+
+    def run():
+        return kernels.gemm(A[0], B[0], 1.5, -0.5, C[0])[None] if batch == 1 else kernels.gemm(A, B, 1.5, -0.5, C)
+
+    D = run()
+    assert torch.equal(D, run())
+    ref = 1.5 * (A.double() @ B.double()) - 0.5 * C.double()
+    den = 1.5 * (A.double().abs() @ B.double().abs()) + 0.5 * C.double().abs()
+    assert ((D.double() - ref).abs() / den).max().item() <= 1e-6
+    # same-sign operands, whose running sums round at every step
+    E = kernels.gemm(A[0].abs(), B[0].abs())
+    want = A[0].double().abs() @ B[0].double().abs()
+    assert ((E.double() - want).abs() / want).max().item() <= 1e-6
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 @pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 2.0**-8), (torch.float16, 2.0**-10)])
 @pytest.mark.parametrize("M,N,K,batch", [(8, 8, 8, 1), (128, 136, 64, 1), (264, 120, 136, 1), (504, 496, 192, 1),
                                          (256, 128, 320, 40), (1784, 2032, 264, 1)])

@@ -466,22 +466,28 @@ __global__ __launch_bounds__(64 * WAVES) void sgemm_direct_kernel(GemmArgs g) {
 }
 
 template <int BM, int BN, int WGM, bool AKC, bool BKC>
-static int run_tile(GemmArgs g, int splits, size_t ws_bytes, hipStream_t s) {
+static int run_tile(GemmArgs g, int splits, hipStream_t s) {
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.N + BN - 1) / BN;
   g.ntiles = g.tiles_m * g.tiles_n * g.batch;
   g.nk = (g.K + 31) / 32;
   g.span = chain_length(g.K, 4) / 32;
   g.splits = splits;
-  if (splits > 1 && (g.ws == nullptr || (size_t)g.ntiles * splits * BM * BN * 4 > ws_bytes))
-    g.splits = 1;
-  if (planned(g, g.splits > 1 ? "sgemm_tile_kernel split" : "sgemm_tile_kernel")) return TRNBLAS_OK;
+  if (g.plan) {
+    static thread_local char name[48];
+    snprintf(name, sizeof name, "sgemm_tile_kernel<%d, %d> in %d", BM, BN, splits);
+    *g.plan = name;
+    return TRNBLAS_OK;
+  }
   hipLaunchKernelGGL((sgemm_tile_kernel<BM, BN, WGM, AKC, BKC>), dim3(g.ntiles * g.splits), dim3(256), 0,
                      s, g);
   int rc = check_launch("trnblas_hip_gemm");
-  if (rc || g.splits == 1) return rc;
-  hipLaunchKernelGGL((sgemm_sum_kernel<BM, BN>), dim3(g.ntiles, BM * BN / 1024), dim3(256), 0, s, g);
-  return check_launch("trnblas_hip_gemm(sum)");
+  if constexpr (BM == 64 && BN == 64) {  // the split tile
+    if (rc || splits == 1) return rc;
+    hipLaunchKernelGGL((sgemm_sum_kernel<BM, BN>), dim3(g.ntiles, BM * BN / 1024), dim3(256), 0, s, g);
+    rc = check_launch("trnblas_hip_gemm(sum)");
+  }
+  return rc;
 }
 
 template <int WAVES, bool AKC, bool BKC, bool SYRK = false>
@@ -522,14 +528,16 @@ static double tiles_of(const GemmArgs& g, int bm, int bn) {
 }
 
 // gemm_dma_kernel (aligned operands): whole rounds of two 128 x 128 tiles per
-// CU, or balanced by narrow tiles / stream-K (choose_sk, narrow_tiles_pay).
+// CU, or balanced by narrow tiles (half the work where N <= 64) / stream-K
+// (choose_sk, narrow_tiles_pay), of which a tile takes up to 63 pieces.
 static double est_dma(const GemmArgs& g) {
   const double cus = device_cus(), t = tiles_of(g, 128, 128), nk = (g.K + 31) / 32;
   const double rounds = std::ceil(t / (2.0 * cus)), eff = t / (rounds * 2.0 * cus);
-  const bool balanced = nk >= 16 && (t <= cus || (eff < 0.9 && rounds <= 8));
-  const double full = t <= cus ? nk : 2.0 * rounds * nk;
-  return 4.1 + 2.32 * (balanced ? t / cus * nk : full) + (balanced ? 9.1 : 0.0) +
-         3.0 * std::max(t / cus, 1.0);
+  const double tail = 3.0 * std::max(t / cus, 1.0);
+  if (nk >= 16 && t <= cus)
+    return 13.2 + std::max(2.32 * 0.5 * tiles_of(g, 128, 64) / cus * nk, 0.65 * nk / 63.0) + tail;
+  if (nk >= 16 && eff < 0.9 && rounds <= 8) return 13.2 + 2.32 * t / cus * nk + tail;
+  return 4.1 + 2.32 * (t <= cus ? nk : 2.0 * rounds * nk) + tail;
 }
 
 // The time of sgemm_direct_kernel for q 32 x 32 tiles per CU of `chunks`
@@ -542,53 +550,65 @@ static double est_direct(int waves, double q, double chunks) {
 enum Kind { kDirect4, kDirect8, kT32x64, kT64x64, kT48x128, kT64x128 };
 
 template <bool AKC, bool BKC>
-static int run(Kind kind, int splits, const GemmArgs& g, size_t ws_bytes, hipStream_t s) {
+static int run(Kind kind, int splits, const GemmArgs& g, hipStream_t s) {
   switch (kind) {
     case kDirect4:
       return run_direct<4, AKC, BKC>(g, s);
     case kDirect8:
       return run_direct<8, AKC, BKC>(g, s);
     case kT32x64:
-      return run_tile<32, 64, 2, AKC, BKC>(g, 1, ws_bytes, s);
+      return run_tile<32, 64, 2, AKC, BKC>(g, 1, s);
     case kT64x64:
-      return run_tile<64, 64, 2, AKC, BKC>(g, splits, ws_bytes, s);
+      return run_tile<64, 64, 2, AKC, BKC>(g, splits, s);
     case kT48x128:
-      return run_tile<48, 128, 1, AKC, BKC>(g, 1, ws_bytes, s);
+      return run_tile<48, 128, 1, AKC, BKC>(g, 1, s);
     default:
-      return run_tile<64, 128, 2, AKC, BKC>(g, 1, ws_bytes, s);
+      return run_tile<64, 128, 2, AKC, BKC>(g, 1, s);
   }
 }
 
-bool sgemm_launch(const GemmArgs& g, bool akc, bool bkc, bool aligned, size_t ws_bytes,
-                  hipStream_t s, int* rc) {
+struct Choice {
+  Kind kind;
+  int splits;
+  double us;
+};
+
+static Choice choose(const GemmArgs& g, size_t ws_bytes) {
   const double nk = (g.K + 31) / 32, chunks = (g.K + 15) / 16;
-  Kind kind = kT64x128;
-  int splits = 1;
-  double best = est_tile({4.2, 0.0, 1.21, 1.53}, tiles_of(g, 64, 128), nk);
+  Choice best{kT64x128, 1, est_tile({4.2, 0.0, 1.21, 1.53}, tiles_of(g, 64, 128), nk)};
   auto take = [&](Kind k, double t, int sp) {
-    if (t < best) {
-      best = t;
-      kind = k;
-      splits = sp;
-    }
+    if (t < best.us) best = Choice{k, sp, t};
   };
   take(kT48x128, est_tile({4.9, 1.09, 0.954, 1.06}, tiles_of(g, 48, 128), nk), 1);
   take(kT32x64, est_tile({3.7, 0.486, 0.322, 0.67}, tiles_of(g, 32, 64), nk), 1);
   const double t64 = tiles_of(g, 64, 64), q32 = tiles_of(g, 32, 32) / device_cus();
   take(kT64x64, est_tile({4.0, 0.737, 0.591, 1.1}, t64, nk), 1);
-  // split along K (at least 8 k-tiles each): the sum kernel's launch, and the
-  // partial tiles' bytes
-  for (int sp = 2; sp <= 16 && 8 * sp <= nk; sp *= 2)
+  // split along K (at least 8 k-tiles each): the sum kernel's launch, the
+  // partial tiles' bytes and its serial reads of one tile's. Fitted (rms 6 %) over 216
+  // products of few tiles, K 2000 to 1200000, up to 512 splits: 63 x 63 x 1000001
+  // 138 us (16 splits 2120)
+  for (int sp = 2; sp <= 512 && 8 * sp <= nk; sp *= 2)
     if (t64 * sp <= 4.0 * device_cus() && t64 * sp * (64 * 64 * 4) <= (double)ws_bytes)
-      take(kT64x64, est_tile({6.1, 0.737, 0.6, 0.0}, t64 * sp, std::ceil(nk / sp)) + t64 * sp * 0.0082,
+      take(kT64x64,
+           est_tile({5.8, 0.741, 0.591, 0.0}, t64 * sp, std::ceil(nk / sp)) + t64 * sp * 0.0048 + sp * 0.073,
            sp);
-  take(kDirect4, est_direct(4, q32, chunks), 1);
-  take(kDirect8, est_direct(8, q32, chunks), 1);
-  if (aligned && est_dma(g) <= best) return false;
+  // (whole-K workgroups: past the fitted K their panels fall out of the caches
+  // together, 10 x (549 x 174 x 41161) 2104 us against 1135 estimated)
+  if (chunks <= 512.0) {
+    take(kDirect4, est_direct(4, q32, chunks), 1);
+    take(kDirect8, est_direct(8, q32, chunks), 1);
+  }
+  return best;
+}
+
+bool sgemm_launch(const GemmArgs& g, bool akc, bool bkc, bool aligned, size_t ws_bytes,
+                  hipStream_t s, int* rc) {
+  const Choice c = choose(g, g.ws ? ws_bytes : 0);
+  if (aligned && est_dma(g) <= c.us) return false;
   if (akc)
-    *rc = bkc ? run<true, true>(kind, splits, g, ws_bytes, s) : run<true, false>(kind, splits, g, ws_bytes, s);
+    *rc = bkc ? run<true, true>(c.kind, c.splits, g, s) : run<true, false>(c.kind, c.splits, g, s);
   else
-    *rc = bkc ? run<false, true>(kind, splits, g, ws_bytes, s) : run<false, false>(kind, splits, g, ws_bytes, s);
+    *rc = bkc ? run<false, true>(c.kind, c.splits, g, s) : run<false, false>(c.kind, c.splits, g, s);
   return true;
 }
 
