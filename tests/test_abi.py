@@ -168,3 +168,14 @@ def test_fp32_gemm_of_few_tiles_and_long_k_is_split():
     assert "direct" not in _plan(F32, 0, 0, 0, 549, 174, 41161, 10)
     # aligned, N <= 64: narrow tiles are half the work
     assert _plan(F32, 0, 0, 1, 66, 3, 33628, 10) == "gemm_dma_kernel narrow"
+
+
+@pytest.mark.parametrize("M,N,K,ta,tb,kernel", [
+    # the larger tiles of the LDS-DMA kernel, also where its last round is half full
+    (6144, 6144, 6144, 0, 1, "gemm_dma_kernel"), (6144, 6144, 6144, 1, 1, "gemm_dma_kernel"),
+    (5620, 5620, 5620, 0, 1, "gemm_dma_kernel"), (1968, 1968, 1968, 0, 1, "gemm_dma_kernel narrow"),
+    # a little over one 32 x 32 tile per CU and a long K: its second round costs a whole one
+    (864, 404, 4940, 1, 0, "gemm_dma_kernel narrow"), (532, 648, 6152, 0, 0, "gemm_dma_kernel narrow"),
+])  # fmt: skip
+def test_aligned_fp32_gemm_stays_on_the_lds_dma_kernel_where_it_is_faster(M, N, K, ta, tb, kernel):
+    assert _plan(F32, 0, ta, tb, M, N, K) == kernel

@@ -529,22 +529,29 @@ static double tiles_of(const GemmArgs& g, int bm, int bn) {
 
 // gemm_dma_kernel (aligned operands): whole rounds of two 128 x 128 tiles per
 // CU, or balanced by narrow tiles (half the work where N <= 64) / stream-K
-// (choose_sk, narrow_tiles_pay), of which a tile takes up to 63 pieces.
+// (choose_sk, narrow_tiles_pay), of which a tile takes up to 63 pieces. Fitted
+// to 330 products' times (rms 7 %) and set against this file's (whose 64 x 64
+// tiles are estimated 10 % high at 1 ms and more) where the two cross.
 static double est_dma(const GemmArgs& g) {
   const double cus = device_cus(), t = tiles_of(g, 128, 128), nk = (g.K + 31) / 32;
+  const double whole = std::floor(t / (2.0 * cus)), left = t - whole * 2.0 * cus;
   const double rounds = std::ceil(t / (2.0 * cus)), eff = t / (rounds * 2.0 * cus);
-  const double tail = 3.0 * std::max(t / cus, 1.0);
-  if (nk >= 16 && t <= cus)
-    return 13.2 + std::max(2.32 * 0.5 * tiles_of(g, 128, 64) / cus * nk, 0.65 * nk / 63.0) + tail;
-  if (nk >= 16 && eff < 0.9 && rounds <= 8) return 13.2 + 2.32 * t / cus * nk + tail;
-  return 4.1 + 2.32 * (t <= cus ? nk : 2.0 * rounds * nk) + tail;
+  if (t <= cus)
+    return nk < 16 ? 7.1 + 2.25 * nk
+                   : 18.0 + std::max(2.18 * 0.5 * tiles_of(g, 128, 64) / cus * nk, 0.65 * nk / 63.0);
+  // (after whole rounds stream-K needs 4 k-tiles or 1 / 63 of K a workgroup)
+  if (nk >= 16 && eff < 0.9 && rounds <= 8 &&
+      (whole == 0.0 || left * nk / (2.0 * cus) >= std::max(4.0, std::ceil(nk / 63.0))))
+    return 30.0 + (2.14 * nk + 3.0) * t / cus;
+  const double last = left == 0.0 ? 0.0 : left <= cus && nk >= 16 ? 1.1 : 2.0;  // tiles per CU
+  return 4.1 + 2.1 * (2.0 * whole + last) * nk + 3.75 * t / cus;
 }
 
 // The time of sgemm_direct_kernel for q 32 x 32 tiles per CU of `chunks`
-// 16-wide chunks.
-static double est_direct(int waves, double q, double chunks) {
-  return waves == 4 ? 3.3 + std::max(0.54 * std::ceil(chunks / 4), 0.104 * q * chunks) + 0.59 * q
-                    : 3.25 + std::max(0.80 * std::ceil(chunks / 8), 0.106 * q * chunks) + 0.95 * q;
+// 16-wide chunks (w: the CU's MFMA time per chunk).
+static double est_direct(int waves, double q, double chunks, double w) {
+  return waves == 4 ? 3.3 + std::max(0.54 * std::ceil(chunks / 4), w * chunks) + 0.59 * q
+                    : 3.25 + std::max(0.80 * std::ceil(chunks / 8), w * chunks) + 0.95 * q;
 }
 
 enum Kind { kDirect4, kDirect8, kT32x64, kT64x64, kT48x128, kT64x128 };
@@ -595,8 +602,10 @@ static Choice choose(const GemmArgs& g, size_t ws_bytes) {
   // (whole-K workgroups: past the fitted K their panels fall out of the caches
   // together, 10 x (549 x 174 x 41161) 2104 us against 1135 estimated)
   if (chunks <= 512.0) {
-    take(kDirect4, est_direct(4, q32, chunks), 1);
-    take(kDirect8, est_direct(8, q32, chunks), 1);
+    // (past 128 chunks the last round costs as much as a full one)
+    const double w = chunks > 128.0 ? 0.095 * rounds_of(q32) : 0.104 * q32;
+    take(kDirect4, est_direct(4, q32, chunks, w), 1);
+    take(kDirect8, est_direct(8, q32, chunks, 1.02 * w), 1);
   }
   return best;
 }
@@ -624,7 +633,7 @@ bool ssyrk_launch(const GemmArgs& g, bool kc, bool aligned, hipStream_t s, int* 
   const double t = (g.M + 31) / 32, chunks = (g.K + 15) / 16;
   const double q = 0.5 * t * (t + 1.0) / device_cus();
   if (aligned ? q > 12.0 || q * chunks > 300.0 || chunks > 192.0 : q > 20.0 || chunks > 256.0) return false;
-  if (est_direct(4, q, chunks) <= est_direct(8, q, chunks))
+  if (est_direct(4, q, chunks, 0.104 * q) <= est_direct(8, q, chunks, 0.106 * q))
     *rc = kc ? run_direct<4, true, true, true>(g, s) : run_direct<4, false, false, true>(g, s);
   else
     *rc = kc ? run_direct<8, true, true, true>(g, s) : run_direct<8, false, false, true>(g, s);
