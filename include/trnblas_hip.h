@@ -126,6 +126,13 @@ int trnblas_hip_pack_k(int dtype, int64_t R, int64_t K, const void* X, int64_t s
                        void* stream);
 
 /*
+ * 1 when packing `elements` elements of an fp32 GEMM's operands (those that
+ * LDS DMA cannot read in place) is expected to make it faster than reading
+ * them in place, else 0. Launches nothing and needs no GPU.
+ */
+int trnblas_hip_gemm_pack_pays(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t elements);
+
+/*
  * SYRK:  D = alpha * op(A) * op(A)^T + beta * sym_uplo(C), returned full.
  *
  * Replaces torch.ops.trnblas.syrk (trnblas/nki/_native.py:124-132; kernel

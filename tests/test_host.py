@@ -651,3 +651,34 @@ def test_syrk_operand_past_32_bit_panel_offsets_is_packed(monkeypatch):
     assert not seen
     k._packed_syrk_operand(A, True, A, True, 16_800_001, 533, 4001)
     assert seen
+
+
+@pytest.mark.parametrize("M,N,K,packs", [
+    (4095, 4095, 4095, True), (3583, 3583, 3583, True), (1258, 1258, 19063, True), (9722, 19004, 205, True),
+    (1535, 1535, 1535, False), (2047, 2049, 2051, False), (48, 442369, 385, False), (17517, 702, 11415, False),
+    (63, 63, 1000001, False),
+])  # fmt: skip
+def test_unaligned_fp32_gemm_is_packed_by_shape(monkeypatch, M, N, K, packs):
+    # where the copy is small against the product (large M and N) or no in-place
+    # kernel splits K well, and not for skinny products of the same work
+    from trnblas_amd.hip import _lib
+    from trnblas_amd.hip import kernels as k
+
+    if not _lib.available():
+        pytest.skip("library not built")
+    seen = []
+    monkeypatch.setattr(k, "_pack_k", lambda X, kp: seen.append(kp) or X)
+    A, B = torch.zeros(1).expand(M, K), torch.zeros(1).expand(K, N)
+    k._packed_operands(A, B, A, False, K, 0, B, False, N, 0, M, N, K, 1)
+    assert bool(seen) == packs
+
+
+def test_fp32_gemm_packing_counts_only_what_is_copied():
+    # 1136 x 11 x 235752: A is ready in place, so that only the 11 columns of B are copied
+    from trnblas_amd.hip import _lib
+    from trnblas_amd.hip import kernels as k
+
+    if not _lib.available():
+        pytest.skip("library not built")
+    assert k.f32_pack_pays(1136, 11, 235752, 1, 11 * 235752)
+    assert not k.f32_pack_pays(1136, 11, 235752, 1, (1136 + 11) * 235752)

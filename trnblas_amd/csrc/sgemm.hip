@@ -621,6 +621,30 @@ bool sgemm_launch(const GemmArgs& g, bool akc, bool bkc, bool aligned, size_t ws
   return true;
 }
 
+// Packing (M + N) K elements moves them twice (at about 4 TB/s) in one or two
+// launches, and the packed product takes gemm_dma_kernel. The copy's share falls
+// with M and N, so that near-cubes pay from 3500 up, skinny products never, and
+// those whose K no kernel here splits well early. Us packed / in place: 1535^3
+// 98 / 77, 3071^3 491 / 485, 4095^3 1091 / 1118, 6143^3 3520 / 3740, 1258 x 1258
+// x 19063 600 / 751, 9722 x 19004 x 205 870 / 928, 17517 x 702 x 11415 2758 /
+// 2540. Short K, whose time is the store of D, is estimated 3 % high in place.
+// Over 285 unaligned products of 2^30 to 2^38 multiply-adds the choice is 0.3 %
+// off the better one on average, at most 10 %.
+extern "C" int trnblas_hip_gemm_pack_pays(int64_t M, int64_t N, int64_t K, int64_t batch,
+                                          int64_t elements) {
+  if (M < 1 || N < 1 || K < 1 || batch < 1 || M >= (1ll << 31) || N >= (1ll << 31) ||
+      K >= (1ll << 31) - 4 || batch >= (1ll << 31))
+    return 0;
+  GemmArgs g{};
+  g.M = (int)M;
+  g.N = (int)N;
+  g.K = (int)K;
+  g.batch = (int)batch;
+  const double in_place = choose(g, trnblas_hip_gemm_workspace()).us;
+  const double packed = est_dma(g) + 6.0 + 8.0 * (double)elements / 4e6;
+  return in_place > (K < 1024 ? 1.03 : 1.0) * packed;
+}
+
 // SYRK of few 128 x 128 tiles: gemm.hip's kernels spend it on instruction
 // fetch and idle CUs, and unaligned operands ran at half the rate. Limits: a
 // wave's serial chain (K to 3072 aligned, 4096 not: past them stream-K over

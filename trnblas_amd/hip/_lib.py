@@ -51,6 +51,7 @@ SIGNATURES = {
         ctypes.c_char_p,
         [_c_int, _c_int, _c_int, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64],
     ),
+    "trnblas_hip_gemm_pack_pays": (_c_int, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64]),
     "trnblas_hip_pack_k": (
         _c_int,
         [_c_int, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64, _c_ptr, _c_i64, _c_i64, _c_i64]

@@ -680,9 +680,9 @@ def gemm_fast(alpha, A, B, beta, C, transA, transB):
     """level3.gemm's common case without the general routing: 2-D fp32
     operands on one GPU, no gradient, the native GEMM policy auto or hip,
     each operand row-major or a transposed row-major view that the kernels
-    read in place (16-byte aligned; ragged leading dimensions and extents below
-    the size from which the general path packs them), C absent or of the result's shape with unit column
-    stride. Returns alpha op(A) op(B) + beta C, or None (the general path
+    read in place (16-byte aligned; ragged leading dimensions and extents where
+    the general path would not pack them), C absent or of the result's shape
+    with unit column stride. Returns alpha op(A) op(B) + beta C, or None (the general path
     then decides, as for every other call; also on a library error, which
     the general path reports). The route is the one `_gemm_route` gives
     these operands ("hip"); the host time per call is about half of the
@@ -736,8 +736,13 @@ def gemm_fast(alpha, A, B, beta, C, transA, transB):
     else:
         return None
     pa, pb = A.data_ptr(), B.data_ptr()
-    if (pa | pb) & 15 or ((lda | ldb | aext | bext) & 3 and M * N * K >= kern._pack_min_macs(4)):
-        return None  # (the latter are packed first)
+    if (pa | pb) & 15:
+        return None
+    if (lda | ldb | aext | bext) & 3:
+        na = M * K if K & 3 or (lda | aext) & 3 else 0
+        nb = N * K if K & 3 or (ldb | bext) & 3 else 0
+        if kern.f32_pack_pays(M, N, K, 1, na + nb):
+            return None
     c, ldc, cb = 0, N, 0.0
     if C is not None and beta != 0.0:
         if (

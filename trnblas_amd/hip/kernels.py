@@ -95,7 +95,7 @@ def _batched_layout(X: torch.Tensor):
 # 16-byte group of an operand lies wholly inside or outside the matrix: a
 # 16-byte aligned base, and a leading dimension, batch stride and contiguous
 # extent that are multiples of 16 bytes. Other operands run on
-# register-staged kernels: fp32 GEMM at any alignment on sgemm.hip's (72-125
+# register-staged kernels: fp32 GEMM at any alignment on sgemm.hip's (77-125
 # TFLOP/s from 1535^3 up), small 16-bit products and SYRKs on 32 x 32 tiles
 # (hgemm.hip, sgemm.hip), the rest at 74 TFLOP/s fp32 SYRK and 81 TFLOP/s
 # bf16 at 4095^3 (737 after packing). From PACK_MIN_MACS multiply-adds per
@@ -103,28 +103,28 @@ def _batched_layout(X: torch.Tensor):
 # K-contiguous buffers whose rows are padded with zeros to a multiple of 16
 # bytes (zero products add nothing to any sum; the reference pads its kernel
 # operands the same way, nki/dispatch.py:2344-2368) and the product takes the
-# DMA kernel. Below it the pack launches cost more than they save. Where the
-# 32 x 32 kernels serve unaligned operands (DIRECT_TILES), packing starts at 4
-# times that size: over random shapes there they are 2.1x faster (batched bf16,
-# none slower, even from 2^30 on: 31 x (175 x 164 x 1098) 41 us packed, 20 in
-# place), 1.4x (fp32 SYRK, none slower; 879 x 2372 47 and 37) and about 2x
-# (16-bit SYRK, M-contiguous; 914 x 814 15.2 and 8.3). K-contiguous 16-bit SYRKs
-# are even (759 x 1139 16.2 and 15.5, 1267 x 411 12.4 and 14.0), and past the
-# limits of DIRECT_TILES packed is up to 1.3x faster (2230 x 89 13 and 16). An
-# fp32 GEMM, whose kernels read any alignment, packs from F32_GEMM_PACK_FACTOR
-# times that size: over random unaligned shapes packing is 1.6x slower than in place at 2^30 multiply-adds,
-# 1.26x at 2^33, 1.12x at 2^36, where cubes are even (4095^3 1100 us packed,
-# 1186 in place).
+# DMA kernel. Below it the pack launches cost more than they save.
+#
+# An fp32 GEMM is packed from there on where trnblas_hip_gemm_pack_pays (the
+# copy and the DMA kernel's estimated time against the in-place kernels')
+# says so: about from 3500^3 on, not at all where M or N is small.
+#
+# Where the 32 x 32 kernels serve unaligned operands (DIRECT_TILES), packing
+# starts at 4 times PACK_MIN_MACS: over random shapes there they are 2.1x faster
+# (batched bf16, none slower, even from 2^30 on: 31 x (175 x 164 x 1098) 41 us
+# packed, 20 in place), 1.4x (fp32 SYRK, none slower; 879 x 2372 47 and 37) and
+# about 2x (16-bit SYRK, M-contiguous; 914 x 814 15.2 and 8.3). K-contiguous
+# 16-bit SYRKs are even (759 x 1139 16.2 and 15.5, 1267 x 411 12.4 and 14.0), and
+# past the limits of DIRECT_TILES packed is up to 1.3x faster (2230 x 89 13 and 16).
 PACK_MIN_MACS = {4: 1 << 30, 2: 1 << 28}
-F32_GEMM_PACK_FACTOR = 64
 # Largest numbers of 32 x 32 tiles (per launch, 256 CUs) of the unaligned 16-bit
 # GEMMs and the fp32 / 16-bit SYRKs (these only M-contiguous) that are packed
-# only later, and the largest k of those SYRKs and
-# of the GEMMs by how many operands are K-contiguous (hgemm_launch's limits of a
-# workgroup's serial chain: past them stream-K over packed operands is faster,
-# 86 x 29 x 168729 621 us in place, 79 packed)
-DIRECT_MAX_K = (12288, 8192, 4096)
+# only later, and the largest k of those SYRKs
 DIRECT_TILES = {"gemm": 12 * 256, "syrk": {4: (20 * 256, 4096), 2: (4 * 256, 2048)}}
+# The largest K of those GEMMs, by how many operands are K-contiguous
+# (hgemm_launch's limits of a workgroup's serial chain: past them stream-K over
+# packed operands is faster, 86 x 29 x 168729 621 us in place, 79 packed)
+DIRECT_MAX_K = (12288, 8192, 4096)
 
 # TRNBLAS_GEMM_RAGGED=0 restores the reference's pad-first path
 # (nki/dispatch.py:144-151, read at import as there): every operand the DMA
@@ -135,10 +135,17 @@ _RAGGED_ENABLED: bool = os.environ.get("TRNBLAS_GEMM_RAGGED", "1").strip().lower
 )  # fmt: skip
 
 
-def _pack_min_macs(elem_size: int, syrk: bool = False) -> int:
-    if not _RAGGED_ENABLED:
-        return 0
-    return PACK_MIN_MACS[elem_size] * (F32_GEMM_PACK_FACTOR if elem_size == 4 and not syrk else 1)
+def _pack_min_macs(elem_size: int) -> int:
+    return PACK_MIN_MACS[elem_size] if _RAGGED_ENABLED else 0
+
+
+def f32_pack_pays(M: int, N: int, K: int, nb: int, elements: int) -> bool:
+    """Whether an fp32 GEMM that LDS DMA cannot serve in place is packed
+    (`elements` of its operands)."""
+    least = _pack_min_macs(4)
+    if least == 0 or nb * M * N * K < least:
+        return least == 0
+    return _lib.available() and bool(_lib.load().trnblas_hip_gemm_pack_pays(M, N, K, nb, elements))
 
 
 def _panel_fits(k_contiguous: bool, ld: int, elem_size: int) -> bool:
@@ -170,12 +177,13 @@ def _packed_operands(A, B, a, ta, lda, sa, b, tb, ldb, sb, M, N, K, nb):
     batch 1 broadcast): (a, ta, lda, sa, b, tb, ldb, sb, K) as laid out, or
     with the operands the DMA kernel cannot read packed K-contiguous (and K
     padded when it is not a multiple of 16 bytes)."""
-    ev = 16 // A.element_size()
-    least = _pack_min_macs(A.element_size())
-    if ev == 8 and nb * -(-M // 32) * -(-N // 32) <= DIRECT_TILES["gemm"] and K <= DIRECT_MAX_K[(not ta) + tb]:
+    es = A.element_size()
+    ev = 16 // es
+    fits = _panel_fits(not ta, lda, es) and _panel_fits(tb, ldb, es)
+    least = _pack_min_macs(es)
+    few = nb * -(-M // 32) * -(-N // 32) <= DIRECT_TILES["gemm"] and K <= DIRECT_MAX_K[(not ta) + tb]
+    if ev == 8 and few and fits:
         least *= 4
-    if not (_panel_fits(not ta, lda, A.element_size()) and _panel_fits(tb, ldb, A.element_size())):
-        least = min(least, PACK_MIN_MACS[A.element_size()])
     if nb * M * N * K < least or M == 0 or N == 0 or K == 0:
         return a, ta, lda, sa, b, tb, ldb, sb, K
     a_ok = _dma_ready(a, lda, sa, M if ta else K, ev)
@@ -183,6 +191,10 @@ def _packed_operands(A, B, a, ta, lda, sa, b, tb, ldb, sb, M, N, K, nb):
     kp = -(-K // ev) * ev
     if a_ok and b_ok:
         return a, ta, lda, sa, b, tb, ldb, sb, K
+    if ev == 4 and fits:
+        na, nbb = (M * K * (A.shape[0] if A.dim() == 3 else 1)), (N * K * (B.shape[0] if B.dim() == 3 else 1))
+        if not f32_pack_pays(M, N, K, nb, na * (kp != K or not a_ok) + nbb * (kp != K or not b_ok)):
+            return a, ta, lda, sa, b, tb, ldb, sb, K
     if kp != K or not a_ok:
         pa = _pack_k(A, kp)
         a, ta, lda, sa = pa, False, kp, (M * kp if pa.dim() == 3 and pa.shape[0] > 1 else 0)
@@ -195,13 +207,12 @@ def _packed_operands(A, B, a, ta, lda, sa, b, tb, ldb, sb, M, N, K, nb):
 def _packed_syrk_operand(A, trans, a, t, lda, n, k):
     """SYRK's (a, t, lda, k) for op(A) (n, k): as laid out, or packed
     K-contiguous with k padded to a multiple of 16 bytes (see _packed_operands)."""
-    ev = 16 // A.element_size()
-    least, tiles = _pack_min_macs(A.element_size(), True), -(-n // 32)
-    most, longest = DIRECT_TILES["syrk"][A.element_size()]
-    if tiles * (tiles + 1) // 2 <= most and k <= longest and (ev == 4 or t):
+    es = A.element_size()
+    ev = 16 // es
+    least, tiles = _pack_min_macs(es), -(-n // 32)
+    most, longest = DIRECT_TILES["syrk"][es]
+    if tiles * (tiles + 1) // 2 <= most and k <= longest and (ev == 4 or t) and _panel_fits(not t, lda, es):
         least *= 4
-    if not _panel_fits(not t, lda, A.element_size()):
-        least = min(least, PACK_MIN_MACS[A.element_size()])
     if n * n * k < least or n == 0 or k == 0 or _dma_ready(a, lda, 0, n if t else k, ev):
         return a, t, lda, k
     kp = -(-k // ev) * ev
