@@ -32,10 +32,9 @@ int check_launch(const char* what);
 int device_cus();
 
 // One diagonal block of the metric Cholesky (metric.hip): trnblas_hip_chol_block,
-// which always clears Linv above its diagonal (zero_upper) and takes diagonals
-// below the normal range (any_scale).
+// which takes diagonals below the normal range (any_scale).
 int chol_block(int64_t nb, double* A, int64_t lda, double* Linv, int64_t ldl, int32_t* info,
-               int64_t offset, bool zero_upper, bool any_scale, hipStream_t stream);
+               int64_t offset, bool any_scale, hipStream_t stream);
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));

@@ -388,12 +388,13 @@ __device__ __forceinline__ void store_lower(const double* G, TT* Z, int64_t zr, 
 // pivots, and 1 / d overflows below 2^-1024: with SCALE, a block with a diagonal
 // element below 2^-960 is factored as 2^120 times itself (a pivot that the
 // updates leave of a larger one is at least its rounding, 2^-53 of it; 1 us
-// more a block: the metric driver scales the whole matrix instead). zero_upper: the sub-blocks
-// of Li above its diagonal ones are cleared (else they hold zeros already).
+// more a block: the metric driver scales the whole matrix instead). The
+// sub-blocks of Li above its diagonal ones are cleared: the triangular products
+// that read it take them as zeros.
 template <bool SCALE>
 __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, int64_t lda,
                                                            double* Li, int64_t ldl, int32_t* info,
-                                                           int offset, int zero_upper) {
+                                                           int offset) {
   constexpr int NW = kThreads / 64;
   __shared__ double G[kNLow * kSB];
   __shared__ double scr[NW][kSB];  // T of the inverse's block row; chol16's exchange
@@ -446,11 +447,9 @@ __global__ __launch_bounds__(kThreads) void chol128_kernel(int nb, double* A, in
     }
 #pragma unroll
     for (int x = 0; x < 5; ++x) store_acc(G + (wave + 7 * x) * kSB, lane, v[x]);
-    if (zero_upper) {
-      for (int x = tid - 64; x < kCholNB * kCholNB; x += kThreads - 64) {
-        const int i = x >> 7, k = x & 127;
-        if ((k >> 4) > (i >> 4) && i < nb && k < nb) Li[(int64_t)i * ldl + k] = 0.0;
-      }
+    for (int x = tid - 64; x < kCholNB * kCholNB; x += kThreads - 64) {
+      const int i = x >> 7, k = x & 127;
+      if ((k >> 4) > (i >> 4) && i < nb && k < nb) Li[(int64_t)i * ldl + k] = 0.0;
     }
   }
   __syncthreads();
@@ -556,8 +555,7 @@ __global__ __launch_bounds__(kThreads) void trinv128_kernel(int n, int upper, in
 using namespace trnblas;
 
 int trnblas::chol_block(int64_t nb, double* A, int64_t lda, double* Linv, int64_t ldl,
-                        int32_t* info, int64_t offset, bool zero_upper, bool any_scale,
-                        hipStream_t stream) {
+                        int32_t* info, int64_t offset, bool any_scale, hipStream_t stream) {
   TRNBLAS_CHECK_ARG(nb >= 0 && nb <= kCholNB, "chol_block: nb %lld not in [0, %d]", (long long)nb,
                     kCholNB);
   if (nb == 0) return TRNBLAS_OK;
@@ -566,14 +564,14 @@ int trnblas::chol_block(int64_t nb, double* A, int64_t lda, double* Linv, int64_
   TRNBLAS_CHECK_ARG(offset >= 0 && offset < (1ll << 30), "chol_block: bad offset");
   auto kern = any_scale ? chol128_kernel<true> : chol128_kernel<false>;
   hipLaunchKernelGGL(kern, dim3(1), dim3(kThreads), 0, stream, (int)nb, A, lda, Linv, ldl, info,
-                     (int)offset, (int)zero_upper);
+                     (int)offset);
   return check_launch("chol_block");
 }
 
 extern "C" int trnblas_hip_chol_block(int64_t nb, double* A, int64_t lda, double* Linv,
                                       int64_t ldl, int32_t* info, int64_t offset, void* stream) {
   clear_error();
-  return chol_block(nb, A, lda, Linv, ldl, info, offset, true, true, (hipStream_t)stream);
+  return chol_block(nb, A, lda, Linv, ldl, info, offset, true, (hipStream_t)stream);
 }
 
 extern "C" int trnblas_hip_tri_inv_blocks(int dtype, int64_t n, int upper, int unit, const void* T,

@@ -217,7 +217,7 @@ extern "C" int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t l
   };
   auto chol = [&](int64_t k) {  // L_bb into W (lower triangle), L_bb^-1 = Y_bb into Y
     return chol_block(n - k < kNB ? n - k : kNB, W + k * npad + k, npad, Y + k * npad + k, npad, info,
-                      k, true, false, main);
+                      k, false, main);
   };
 
   // up to two steps there is no trailing update, and the hand-overs to the
