@@ -102,8 +102,9 @@ def test_syrk_triangle(dev, n, k, trans, uplo):
      (130, 70, 20000, False, True)],
 )
 def test_gemm_stream_k_splits(dev, M, N, K, ta, tb):
-    # shapes whose tiles underfill the GPU: the k-iterations are split over
-    # many workgroups and summed by the fixup kernel (several-way splits)
+    # shapes whose tiles underfill the GPU: K is split over several workgroups a
+    # tile and summed (but for the one that fills it: test_gemm_lds_dma_kernels
+    # has the stream-K kernels)
     from trnblas_amd.hip import kernels
 
     g = torch.Generator().manual_seed(M + K)
@@ -140,10 +141,9 @@ def test_syrk_stream_k(dev, n, k, uplo):
 @pytest.mark.parametrize("n,k", [(384, 200), (300, 77)])
 @pytest.mark.parametrize("uplo", ["lower", "upper"])
 def test_syrk_16bit(dev, dtype, tol, n, k, uplo):
-    # 16-bit SYRK: (384, 200) runs the direct-to-LDS kernel with whole
-    # interior tiles (vector mirrored stores of 8 bytes), (300, 77) the
-    # register-staged kernel with ragged edges. The only rounding beyond
-    # fp32 accumulation is the final one to the 16-bit output.
+    # 16-bit SYRK on 32 x 32 tiles, aligned (384, 200) and with ragged edges (300,
+    # 77; test_syrk_kernels has the other kernels). The only rounding beyond fp32
+    # accumulation is the final one to the 16-bit output.
     from trnblas_amd.hip import kernels
 
     g = torch.Generator().manual_seed(n * 7 + k)
@@ -241,8 +241,7 @@ def test_syrk_unaligned_c_ld(dev):
 
 @pytest.mark.parametrize("M,N,K", [(128, 128, 32768), (256, 128, 20000), (1024, 1024, 1024), (64, 300, 4096)])
 def test_gemm_stream_k_few_tiles(dev, M, N, K):
-    # a handful of tiles with long K: every tile is split over many
-    # workgroups (up to the fixup's 64 contributors per tile)
+    # a handful of tiles with long K: K is split over many workgroups a tile
     from trnblas_amd.hip import kernels
 
     g = torch.Generator().manual_seed(M + N + K)
@@ -414,10 +413,9 @@ def test_syrk_16bit_trans_aligned(dev, dtype, tol):
 )
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
 def test_gemm_narrow_tiles(dev, batch, M, N, K, ta, tb):
-    # launches whose 128 x 128 tiles fill at most one slot per CU of the
-    # MI355X's 256 CUs run the 128 x 64 kernel: whole tiles where they fill
-    # one round of two slots per CU, else split by stream-K over 128 x 64
-    # tiles (up to the fixup's 64 contributors at K = 30000): every layout,
+    # aligned products whose 128 x 128 tiles fill at most one slot per CU of the
+    # MI355X's 256 CUs, on whichever kernel serves them (two of these sizes the
+    # 128 x 64 tiles; test_gemm_lds_dma_kernels names its kernel): every layout,
     # ragged edges, a batch, alpha / beta, at the 1e-6 gate
     from trnblas_amd.hip import kernels
 
@@ -466,7 +464,8 @@ def test_gemm_pipe_kernel_transposed_a(dev, batch, M, N, K):
 def test_gemm_16bit_narrow_tiles(dev, dtype, tol, M, N, K, ta, tb):
     # 16-bit launches with at most one 128 x 128 tile per CU and >= 20
     # 64-wide k-tiles run the 128 x 64 kernel (stream-K where the grid is
-    # small); every layout, a ragged edge, against fp64 of the rounded inputs
+    # small), 1280 x 1272 x 1280 hgemm128_kernel; every layout, a ragged edge,
+    # against fp64 of the rounded inputs
     from trnblas_amd.hip import kernels
 
     g = torch.Generator().manual_seed(M + N + K + 2 * ta + tb)
@@ -533,17 +532,21 @@ def test_gemm_packed_operands(dev, monkeypatch, dtype, tol, batch, bb, M, N, K, 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-6), (torch.bfloat16, 2.0**-8)])
 @pytest.mark.parametrize("M,N,K,ta,tb", [(1537, 1539, 1541, False, False), (2047, 1025, 1027, True, True),
                                          (1023, 2049, 1031, False, True)])
-def test_gemm_unaligned_large(dev, dtype, tol, M, N, K, ta, tb):
-    # products above the packing threshold with odd extents take the DMA
-    # kernel on packed operands (at the default threshold)
+def test_gemm_unaligned_large(dev, monkeypatch, dtype, tol, M, N, K, ta, tb):
+    # products above the packing threshold with odd extents: 16-bit ones take the
+    # DMA kernel on packed operands, fp32 ones of these sizes are read in place
     from trnblas_amd.hip import kernels
 
     assert M * N * K >= kernels.PACK_MIN_MACS[4]
+    packs = []
+    orig = kernels._pack_k
+    monkeypatch.setattr(kernels, "_pack_k", lambda X, kp: packs.append(kp) or orig(X, kp))
     g = torch.Generator().manual_seed(M + N + K)
     A = (torch.randn(K, M, generator=g).T if ta else torch.randn(M, K, generator=g)).to(dtype)
     B = (torch.randn(N, K, generator=g).T if tb else torch.randn(K, N, generator=g)).to(dtype)
     C = torch.randn(M, N, generator=g).to(dtype)
     D = kernels.gemm(A.to(dev), B.to(dev), 1.0, 0.5, C.to(dev)).cpu()
+    assert bool(packs) == (dtype != torch.float32)
     ref = A.double() @ B.double() + 0.5 * C.double()
     den = A.double().abs() @ B.double().abs() + 0.5 * C.double().abs()
     assert ((D.double() - ref).abs() / den).max().item() <= tol
@@ -664,9 +667,10 @@ def test_sgemm_many_splits(dev, M, N, K, batch, ta, tb):
 @pytest.mark.parametrize("M,N,K,batch", [(8, 8, 8, 1), (128, 136, 64, 1), (264, 120, 136, 1), (504, 496, 192, 1),
                                          (256, 128, 320, 40), (1784, 2032, 264, 1)])
 def test_one_round_16bit(dev, dtype, tol, M, N, K, batch, ta, tb):
-    # hgemm128_kernel (up to one 128 x 128 tile per CU): 1..6 k-tiles against its
-    # four LDS stages, ragged tile edges and K tails, batches, against fp64 at
-    # the 16-bit gate (one rounding of |A||B| + |C|)
+    # up to one 128 x 128 tile per CU: the last size on hgemm128_kernel (its other
+    # k-tile counts in test_hgemm128_k_tiles), the others on 32 x 32 tiles; ragged
+    # tile edges and K tails, batches, against fp64 at the 16-bit gate (one
+    # rounding of |A||B| + |C|)
     from trnblas_amd.hip import kernels
 
     g = torch.Generator().manual_seed(M + N + K)
@@ -740,6 +744,110 @@ def test_syrk_small_tiles(dev, n, k, uplo, trans, dtype):
     D = kernels.syrk(A, 1.5, -0.5, C, trans=trans, uplo=uplo)
     assert torch.equal(D, D.mT)
     Ad = (A.mT if trans else A).double()
+    ref = 1.5 * (Ad @ Ad.mT) - 0.5 * Cs
+    den = 1.5 * (Ad.abs() @ Ad.abs().mT) + 0.5 * Cs.abs()
+    eps = 0.0 if dtype == torch.float32 else torch.finfo(dtype).eps
+    tiny = torch.finfo(dtype).tiny * torch.finfo(dtype).eps
+    assert ((D.double() - ref).abs() <= 0.5 * eps * ref.abs() + (1 + eps) * 1e-6 * den + tiny).all()
+
+
+def _plan(dtype, M, N, K, ta=False, tb=False, batch=1, syrk=False, lda=None, ldb=None):
+    """The kernel that serves a product of these sizes (operands at 16-byte aligned bases)."""
+    from trnblas_amd.hip import _lib
+
+    lda, ldb = lda or (M if ta else K), ldb or (K if tb else N)
+    code = _lib.DTYPE_CODES[dtype]
+    return _lib.load().trnblas_hip_gemm_plan(code, int(syrk), int(ta), int(tb), M, N, K, lda, ldb, batch).decode()
+
+
+def _check_gemm(dev, dtype, kernel, batch, M, N, K, ta, tb):
+    """kernels.gemm with alpha and beta on the kernel named, twice the same bits,
+    against fp64: fp32 sums (1e-6 |A||B| + |C|) and one rounding to the type."""
+    from trnblas_amd.hip import kernels
+
+    assert _plan(dtype, M, N, K, ta, tb, batch).startswith(kernel)
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 7 * K + 2 * ta + tb)
+    A = torch.randn(batch, *((K, M) if ta else (M, K)), generator=g, device=dev).to(dtype)
+    B = torch.randn(batch, *((N, K) if tb else (K, N)), generator=g, device=dev).to(dtype)
+    A, B = (A.mT if ta else A), (B.mT if tb else B)
+    C = torch.randn(batch, M, N, generator=g, device=dev).to(dtype)
+
+    def run():
+        return kernels.gemm(A[0], B[0], 1.5, -0.5, C[0])[None] if batch == 1 else kernels.gemm(A, B, 1.5, -0.5, C)
+
+    D = run()
+    assert torch.equal(D, run())
+    Ad, Bd = A.double().contiguous(), B.double().contiguous()
+    ref = 1.5 * (Ad @ Bd) - 0.5 * C.double()
+    den = 1.5 * (Ad.abs() @ Bd.abs()) + 0.5 * C.double().abs()
+    eps = 0.0 if dtype == torch.float32 else torch.finfo(dtype).eps
+    tiny = torch.finfo(dtype).tiny * torch.finfo(dtype).eps
+    assert ((D.double() - ref).abs() <= 0.5 * eps * ref.abs() + (1 + eps) * 1e-6 * den + tiny).all()
+
+
+LAYOUTS = [(False, False), (True, False), (False, True), (True, True)]
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize(
+    "kernel,batch,M,N,K",
+    # 128 x 64 tiles: whole (N ragged), and split by stream-K, with a batch; 128 x
+    # 128: stream-K alone, stream-K after a whole round, whole rounds (short K)
+    [("gemm_dma_kernel narrow", 1, 1536, 1544, 1536), ("gemm_dma_kernel narrow", 1, 520, 1016, 9000),
+     ("gemm_dma_kernel narrow", 1, 1300, 1280, 5000), ("gemm_dma_kernel narrow", 3, 712, 520, 4096),
+     ("gemm_dma_kernel", 1, 2304, 2400, 1800), ("gemm_dma_kernel", 1, 2900, 3000, 2100),
+     ("gemm_dma_kernel", 2, 2176, 2080, 1500), ("gemm_dma_kernel", 1, 4080, 4092, 260)],
+)  # fmt: skip
+def test_gemm_lds_dma_kernels(dev, kernel, batch, M, N, K, ta, tb):
+    _check_gemm(dev, torch.float32, kernel, batch, M, N, K, ta, tb)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [8, 64, 128, 192, 200, 256, 384])
+def test_hgemm128_k_tiles(dev, dtype, K, ta, tb):
+    # hgemm128_kernel with 1 to 6 k-tiles against its four LDS stages and the two its
+    # movers run ahead, whole and cut last k-tiles, ragged tile edges
+    _check_gemm(dev, dtype, "hgemm128_kernel", 1, 1784, 2032, K, ta, tb)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kernel,batch,M,N,K", [
+    # few tiles and a long K: narrow tiles split into up to 63 pieces, and the
+    # register-staged kernel where operands are unaligned; many small unaligned ones
+    ("gemm_dma_kernel narrow", 1, 64, 64, 65536), ("gemm_dma_kernel narrow", 4, 8, 32, 20000),
+    ("gemm_kernel", 1, 35, 29, 13001), ("gemm_kernel", 1, 131, 257, 16387), ("gemm_kernel", 200, 99, 101, 33),
+])  # fmt: skip
+def test_16bit_gemm_long_k_and_large_batches(dev, dtype, kernel, batch, M, N, K, ta, tb):
+    _check_gemm(dev, dtype, kernel, batch, M, N, K, ta, tb)
+
+
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("uplo", ["lower", "upper"])
+@pytest.mark.parametrize("dtype,kernel,n,k", [
+    (torch.float32, "gemm_dma_kernel", 700, 4096), (torch.float32, "gemm_kernel", 131, 4099),
+    (torch.float32, "gemm_kernel", 3267, 35), (torch.bfloat16, "gemm_dma_kernel", 1032, 4104),
+    (torch.bfloat16, "gemm_dma_kernel", 2600, 136), (torch.float16, "gemm_dma_kernel", 72, 8200),
+    (torch.bfloat16, "gemm_kernel", 131, 8201), (torch.float16, "gemm_kernel", 385, 8209),
+])  # fmt: skip
+def test_syrk_kernels(dev, dtype, kernel, n, k, uplo, trans):
+    # SYRK past the 32 x 32 kernels: LDS DMA (split along K or not) and, unaligned,
+    # the register-staged kernel; both triangles bit-equal, only the referenced
+    # triangle of C read, against fp64
+    from trnblas_amd.hip import kernels
+
+    assert _plan(dtype, n, n, k, ta=trans, syrk=True).startswith(kernel)
+    g = torch.Generator(device=dev).manual_seed(n + 5 * k)
+    A = torch.randn(*((k, n) if trans else (n, k)), generator=g, device=dev).to(dtype)
+    X = torch.randn(n, n, generator=g, device=dev).to(dtype)
+    Cs = (torch.tril(X) + torch.tril(X, -1).mT).double()
+    tri = torch.ones(n, n, device=dev, dtype=torch.bool)
+    tri = torch.tril(tri) if uplo == "lower" else torch.triu(tri)
+    C = torch.where(tri, Cs.to(dtype), torch.full_like(X, float("nan")))
+    D = kernels.syrk(A, 1.5, -0.5, C, trans=trans, uplo=uplo)
+    assert torch.equal(D, D.mT)
+    Ad = (A.mT if trans else A).double().contiguous()
     ref = 1.5 * (Ad @ Ad.mT) - 0.5 * Cs
     den = 1.5 * (Ad.abs() @ Ad.abs().mT) + 0.5 * Cs.abs()
     eps = 0.0 if dtype == torch.float32 else torch.finfo(dtype).eps

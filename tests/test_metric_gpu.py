@@ -48,7 +48,9 @@ def test_trsm_device_bf16_and_views(dev):
     assert np.abs(Xb.double().cpu().numpy() - want).max() < 3e-2 * np.abs(want).max()
 
 
-@pytest.mark.parametrize("n", [1, 2, 127, 129, 1024])
+# (from 513 on the trailing updates and the inverse run on streams of their own, in
+# steps of two 128-wide blocks: last steps of one block, of two, and ragged ones)
+@pytest.mark.parametrize("n", [1, 2, 127, 129, 513, 641, 700, 897, 1024, 1153])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_metric_inv_half_device(dev, n, dtype):
     J = torch.from_numpy(om.spd(n, seed=60 + n))
@@ -127,7 +129,7 @@ def test_chol_block_info(dev):
     assert int(info) == 7
 
 
-@pytest.mark.parametrize("n", [300, 385])
+@pytest.mark.parametrize("n", [300, 385, 700])
 @pytest.mark.parametrize("cond", [1e2, 1e8])
 def test_metric_inv_half_blocked_conditioning(dev, n, cond):
     # several 128-wide blocks, a ragged last one, and RI-like conditioning:
@@ -265,3 +267,33 @@ def test_metric_scale_at_the_ends_of_the_range(dev, n, exp):
         assert int(info) == 0
         got = torch.ldexp(Li.mT, torch.tensor(exp // 2, device=dev))
         assert float((got - want).abs().max()) <= tol * float(want.abs().max())
+
+
+@pytest.mark.parametrize("n,at", [(897, 520), (897, 896), (641, 255), (1153, 1100)])
+def test_metric_error_after_side_stream_updates(dev, n, at):
+    # a pivot that only the updates of earlier blocks make non-positive
+    from trnblas_amd.hip import kernels
+
+    J = torch.from_numpy(om.spd(n, seed=n)).to(dev)
+    J[at, at] = -1.0
+    assert int(kernels.metric_inv_half(J)[1]) == at + 1
+
+
+@pytest.mark.parametrize("n", [641, 897, 1024])
+def test_metric_repeated_and_on_two_streams(dev, n):
+    # the device's side streams are shared: calls in a row and from two caller
+    # streams give the bits of the first
+    from trnblas_amd.hip import kernels
+
+    J = [torch.from_numpy(om.spd(n, seed=s)).to(dev) for s in (1, 2)]
+    want = [kernels.metric_inv_half(j)[0] for j in J]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    got = []
+    for _ in range(3):
+        for s, j in zip(streams, J):
+            with torch.cuda.stream(s):
+                got.append(kernels.metric_inv_half(j)[0])
+    torch.cuda.synchronize()
+    for i, X in enumerate(got):
+        assert torch.equal(X, want[i % 2])
