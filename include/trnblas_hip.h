@@ -515,17 +515,18 @@ int trnblas_hip_dgemm(int transA, int transB, int64_t M, int64_t N, int64_t K, d
  * triangular. Replaces `nki_metric_inv_half` (trnblas/nki/dispatch.py:
  * 1883-1905; its device route `_device_inv_chol_factor` :1866-1870 is
  * torch.linalg.cholesky + the blocked trsm against the identity). One call
- * issues the whole sequence: a right-looking blocked Cholesky (128-wide
- * blocks; trnblas_hip_chol_block on the diagonal, trnblas_hip_dgemm panels
- * and lower-triangle trailing updates, the trailing update on a second
- * stream of the same device so the next diagonal block runs beside it),
- * then L^-1 by recursive doubling over block halves and its transpose.
+ * issues the whole sequence: a right-looking blocked Cholesky in steps of 256
+ * columns (two 128-wide diagonal blocks, each factored and inverted by one
+ * kernel; trnblas_hip_dgemm panels and lower-triangle trailing updates, the
+ * trailing update on a second stream of the same device so the next diagonal
+ * blocks run beside it), the rows of L^-1 behind it on a third stream (one
+ * stream up to n = 512), and the transpose.
  * With J[0] below 2^-960 the whole of J is factored as 2^120 times itself;
  * else a pivot below 2^-1024 counts as not positive.
  * info (device int32) is set to the order of the first leading minor that
  * is not positive definite, else 0 (X is then garbage). workspace: at least
  * trnblas_hip_metric_inv_half_workspace(n) bytes, 256-byte aligned. Calls on
- * one device share its second stream and are serialised on the host.
+ * one device share these streams and are serialised on the host.
  */
 size_t trnblas_hip_metric_inv_half_workspace(int64_t n);
 int trnblas_hip_metric_inv_half(int64_t n, const double* J, int64_t ldj, double* X, int64_t ldx,

@@ -264,12 +264,12 @@ static int run_direct(int waves, GemmArgs g, hipStream_t s) {
 // 47. Both operands K-contiguous read 32 rows at once, words of odd rows five
 // at a time, so these limits are lower (aligned 80 x 4416 SYRK 17.8 us here, 12.6
 // there; unaligned 58 x 7427 37.8 and 27.4).
-// Over 707 random GEMMs and 64 SYRKs (bf16, fp16; M, N, K 1 .. 4096, batches
-// to 64) against gemm.hip's kernels: aligned 1.70x and 2.0x faster on average,
-// unaligned 2.85x and 2.7x, none slower. GPU time (us) before / after, the
-// layouts mixed: 64 x 267 x 892 19.4 / 5.2, 981 x 1109 x 307 41.4 / 11.6, 33 x
-// (518 x 106 x 197) 24.3 / 10.8, 119 x 892 x 2812 29.5 / 10.2; aligned 913 x
-// 224 x 408 9.0 / 5.5. Four waves or eight: the smaller of two fitted times
+// Over 1500 random products (bf16, M and N 8 .. 3000, K 32 .. 20000, batches
+// to 64, the layouts mixed), those past the rule among them, against gemm.hip's
+// kernels (packed where those need it): GEMM 1.65x aligned and 2.5x unaligned
+// faster on average, SYRK 1.65x and 2.3x, one 7 % and one 6 % slower. GPU time (us)
+// before / after: 64 x 267 x 892 (A^T B) 19.9 / 5.3, 33 x (518 x 106 x 197) 28.6 /
+// 13.4, aligned 913 x 224 x 408 (A B^T) 11.3 / 5.6. Four waves or eight: the smaller of two fitted times
 // (rms 15 %; within 0.5 % of the better one on average).
 template <typename T, bool SYRK>
 bool hgemm_launch(const GemmArgs& g, bool akc, bool bkc, bool aligned, hipStream_t s, int* rc) {

@@ -29,8 +29,8 @@
 //     inverts it (chol16: no memory access on its column chain); the other
 //     waves meanwhile apply the rest of the trailing update and form block
 //     row p of the inverse, Y_pj = -Y_pp sum_k L_pk Y_kj.
-// L and Y go to memory from the registers they are formed in. 27 us a
-// block under the tracer (46 us with the diagonal sub-block's columns exchanged through LDS,
+// L and Y go to memory from the registers they are formed in. 25.4 us a
+// block under the tracer (45.4 us with the diagonal sub-block's columns exchanged through LDS,
 // its factorisation and the trailing update one after the other, and the
 // inverse by recursive doubling after all of them).
 // trinv128: the 8 diagonal sub-blocks inverted at once (inv16), then

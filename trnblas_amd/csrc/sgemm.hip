@@ -649,10 +649,11 @@ extern "C" int trnblas_hip_gemm_pack_pays(int64_t M, int64_t N, int64_t K, int64
 // fetch and idle CUs, and unaligned operands ran at half the rate. Limits: a
 // wave's serial chain (K to 3072 aligned, 4096 not: past them stream-K over
 // more CUs is faster) and, aligned, q chunks <= 300, past which the LDS-DMA
-// kernel's fewer L2 bytes count. Over 133 random SYRKs (n to 4096, k to 8192)
-// 2.25x faster on average, none slower. GPU time (us), n x k, before / after:
-// 125 x 160 17.3 / 4.9, 241 x 357 (unaligned) 61.9 / 6.5, 1072 x 116 26.6 /
-// 7.9, 506 x 2606 (unaligned) 35.2 / 21.9.
+// kernel's fewer L2 bytes count. Over 300 random SYRKs (n to 5000, k to 12000, those
+// past the limits among them) 1.75x faster aligned and 2.5x unaligned on average,
+// one 4 % slower. GPU time (us), n x k, before / after: 125 x 160 17.3 / 4.9, 241
+// x 357 (unaligned) 50.8 / 6.6, 1072 x 116 (A^T A) 17.5 / 7.8, 506 x 2606
+// (unaligned) 35.2 / 21.9.
 bool ssyrk_launch(const GemmArgs& g, bool kc, bool aligned, hipStream_t s, int* rc) {
   const double t = (g.M + 31) / 32, chunks = (g.K + 15) / 16;
   const double q = 0.5 * t * (t + 1.0) / device_cus();

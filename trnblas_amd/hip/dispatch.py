@@ -354,12 +354,14 @@ def _dma_ready_2d(X: torch.Tensor, rows_ext: int, cols_ext: int) -> bool:
 
 
 # 16-bit 2-D products whose operands the DMA kernel cannot read in place,
-# below the hipBLASLt bucket above: the register-staged kernel, or packing
-# plus the DMA kernel, against hipBLASLt (bf16, square, measured on the
-# MI355X): 255^3 38 / 30 / 50 us, 511^3 29 / 32 / 23, 767^3 38 / 34 / 28,
-# 1023^3 51 / 40 / 27, 1535^3 111 / 52 / 45. From 2^26 multiply-adds on they
-# go to hipBLASLt; below it hgemm.hip's 32 x 32 kernel now serves them (64 x
-# 267 x 892 5 us on the GPU, 19 on the register-staged kernel).
+# below the hipBLASLt bucket above: from 2^26 multiply-adds on they go to
+# hipBLASLt, below it to hgemm.hip's 32 x 32 kernel (64 x 267 x 892 5 us on
+# the GPU, 11 by hipBLASLt). On the GPU the kernel / hipBLASLt take (bf16, A B,
+# us) 255^3 4.0 / 36.7, 383^3 5.0 / 7.3, 511^3 5.6 / 8.0, 639^3 8.6 / 8.7, 767^3
+# 12.2 / 11.2, 1023^3 18.0 / 12.7, 1535^3 39 / 27 (packed from 1023^3 on); the
+# line was drawn against the register-staged kernel that served them before, and
+# products between it and about 2^28, or skinny ones (119 x 892 x 2812 7.9 /
+# 15.0), would be faster on the kernel.
 _ATEN_16BIT_UNREADY_MIN_MACS = 1 << 26
 
 
@@ -885,12 +887,12 @@ def _trsm_hip(A, B, side, uplo, trans, diag, alpha):
 
 def _metric_inv_half_blocked(J: torch.Tensor) -> torch.Tensor:
     """X = L^-T of a real SPD J on the ROCm device, in fp64, by the native
-    driver trnblas_hip_metric_inv_half: a right-looking blocked Cholesky
-    (128-wide diagonal blocks factored and inverted by one kernel each,
-    fp64 MFMA GEMM panels and lower-triangle trailing updates, the trailing
-    update on a second stream beside the next diagonal block), then L^-1 by
-    recursive doubling over block halves, one batched GEMM pair per level,
-    and its transpose. Returns float64."""
+    driver trnblas_hip_metric_inv_half: a right-looking blocked Cholesky in
+    steps of 256 columns (two 128-wide diagonal blocks, each factored and
+    inverted by one kernel, fp64 MFMA GEMM panels and lower-triangle trailing
+    updates, these on a second stream beside the next diagonal blocks), the
+    rows of L^-1 behind it on a third stream, and the transpose. Returns
+    float64."""
     from . import kernels
 
     X, info = kernels.metric_inv_half(J.to(torch.float64))
@@ -910,7 +912,7 @@ def _metric_solve_route(J: torch.Tensor) -> str:
     `_metric_solve_route`, nki/dispatch.py:1833-1849, and its
     TRNBLAS_METRIC_SOLVE=auto|host|device override). "auto" keeps a device J
     on the device at every size: on the MI355X the fp64 HIP driver beats the
-    host's LAPACK from the smallest metrics up (naux 4096: 2.8 ms against
+    host's LAPACK from the smallest metrics up (naux 4096: 2.2 ms against
     139-217 ms), where the reference's Trainium route sends naux <= 1024 to
     the host. "host" computes the factor with host LAPACK in fp64 and copies
     it back. A host J takes host LAPACK whatever the setting."""
