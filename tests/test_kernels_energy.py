@@ -286,3 +286,10 @@ def test_pair_energy_walks_agree(dev, nocc, nvir, naux):
     e = kernels.pair_energies(B, B, eo, eo, ev, i.int(), j.int(), math="fp16x3").cpu()
     want = float((e * torch.where(i == j, 1.0, 2.0)).sum())
     assert abs(got - want) <= 1e-13 * abs(want)
+
+
+@pytest.mark.parametrize("ic,nocc,nvir", [(2, 3, 6), (1, 2, 31), (2, 2, 32), (1, 3, 33), (3, 250, 33), (1, 2, 95),
+                                          (1, 1, 256), (1, 2, 257), (1, 1, 321)])  # fmt: skip
+def test_mp2_energy_tile_sizes(dev, ic, nocc, nvir):
+    # 32 x 32 tiles up to nvir 256 and 64 x 64 past it, at the edges of both
+    test_mp2_energy_partials_edges(dev, ic, nocc, nvir)

@@ -1403,15 +1403,20 @@ __global__ __launch_bounds__(512, 1) void pair_energy_quad_kernel(PairArgs g) {
 
 // MP2 energy of a precomputed amplitude block (the `mp2_energy` surface,
 // trnblas/nki/dispatch.py:4356-4491), bound by the one read of T from HBM.
-// T_ij is walked in 64 x 64 tile pairs (A <= B): T[B,A] goes through LDS and
+// T_ij is walked in NB x NB tile pairs (A <= B): T[B,A] goes through LDS and
 // is read transposed against T[A,B], which stays in the registers it was
-// loaded into, so every amplitude is read once. A group of 16 lanes reads
-// the 256 bytes of a tile row as 16-byte loads (4-byte aligned: any nvir and
-// ldt), and the next tile pair's loads are in flight behind the current
-// one's arithmetic. A pitch of 65 floats puts the transposed reads of a wave
-// on distinct banks. fp64 terms, fixed-order sums. 16 x 64 pairs of nvir 448
-// (822 MB): 196 us, 4.2 TB/s (646 us with 32 x 32 tiles, 4-byte loads, both
-// tiles through LDS and no load in flight behind the arithmetic).
+// loaded into, so every amplitude is read once. A group of NB / 4 lanes reads
+// a tile row as 16-byte loads (4-byte aligned: any nvir and ldt), and the next
+// tile pair's loads are in flight behind the current one's arithmetic. A pitch
+// of NB + 1 floats spreads the transposed reads of a wave over the banks. fp64
+// terms, fixed-order sums. 16 x 64 pairs of nvir 448 (822 MB): 196 us, 4.2 TB/s
+// (646 us with 32 x 32 tiles, 4-byte loads, both tiles through LDS and no load
+// in flight behind the arithmetic).
+//
+// NB 32 up to nvir 256, where 64 x 64 tiles are padding for the most part (64 x
+// 256 pairs of 20 72 us in 64s, 30 in 32s, 38 before; of 33 91 / 61 / 83; 64 x 64
+// pairs of 200 231 / 190); past it the rows of 256 bytes count, the more so where
+// nvir splits cache lines (16 x 64 pairs of 447 232 / 250, 8 x 64 of 700 268 / 297).
 //
 // A workgroup takes tile pairs split, split + nsplit, ... of one (i, j) pair
 // and writes one partial, so that few pairs still fill the chip.
@@ -1423,16 +1428,19 @@ struct Mp2Args {
   double* out;  // [npairs][nsplit]
 };
 
+constexpr int kMp2SmallNvir = 256;
+
 typedef f32x4 __attribute__((aligned(4))) f32x4u;  // 16-byte access, 4-byte aligned
 
+template <int NB>
 __global__ __launch_bounds__(256) void mp2_energy_kernel(Mp2Args g) {
-  constexpr int NB = 64, P = NB + 1;
+  constexpr int P = NB + 1, RL = NB / 4, RS = 256 / RL, NU = NB / RS;  // lanes of a row, rows a pass
   __shared__ float y[NB * P];
   __shared__ double red[4];
   const int nvir = g.nvir;
   const int pair = blockIdx.x % g.npairs, split = blockIdx.x / g.npairs;
   const int i = pair / g.nocc, j = pair - i * g.nocc;
-  const int c4 = 4 * (threadIdx.x & 15), r0 = threadIdx.x >> 4;  // rows r0 + 16 u
+  const int c4 = 4 * (threadIdx.x % RL), r0 = threadIdx.x / RL;  // rows r0 + RS u
   const double eo = (double)g.eo_chunk[i] + (double)g.eo_full[j];
   const float* Tij = g.T + (int64_t)i * nvir * g.ldt + (int64_t)j * nvir;
   const int nb = (nvir + NB - 1) / NB, items = nb * (nb + 1) / 2;
@@ -1444,12 +1452,12 @@ __global__ __launch_bounds__(256) void mp2_energy_kernel(Mp2Args g) {
     while ((B + 1) * (B + 2) / 2 <= q) ++B;
     A = q - B * (B + 1) / 2;
   };
-  // rows R * 64 + r0 + 16 u, columns C * 64 + c4 .. + 3 (zeros outside)
-  auto load = [&](int R, int C, f32x4(&v)[4]) __attribute__((always_inline)) {
+  // rows R * NB + r0 + RS u, columns C * NB + c4 .. + 3 (zeros outside)
+  auto load = [&](int R, int C, f32x4(&v)[NU]) __attribute__((always_inline)) {
     const int c = C * NB + c4;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int r = R * NB + r0 + 16 * u;
+    for (int u = 0; u < NU; ++u) {
+      const int r = R * NB + r0 + RS * u;
       const float* p = Tij + (int64_t)r * g.ldt + c;
       v[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       if (r < nvir && c + 3 < nvir) {
@@ -1462,7 +1470,7 @@ __global__ __launch_bounds__(256) void mp2_energy_kernel(Mp2Args g) {
     }
   };
   double sum = 0.0;
-  f32x4 xn[4], yn[4];
+  f32x4 xn[NU], yn[NU];
   int A = 0, B = 0;
   if (split < items) {
     tile(split, A, B);
@@ -1470,13 +1478,13 @@ __global__ __launch_bounds__(256) void mp2_energy_kernel(Mp2Args g) {
     load(B, A, yn);
   }
   for (int q = split; q < items; q += g.nsplit) {
-    f32x4 x[4];
+    f32x4 x[NU];
     __syncthreads();  // the last tile pair's reads of y are done
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < NU; ++u) {
       x[u] = xn[u];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) y[(r0 + 16 * u) * P + c4 + e] = yn[u][e];
+      for (int e = 0; e < 4; ++e) y[(r0 + RS * u) * P + c4 + e] = yn[u][e];
     }
     __syncthreads();
     const int a0 = A * NB + r0, b0 = B * NB + c4;
@@ -1490,15 +1498,15 @@ __global__ __launch_bounds__(256) void mp2_energy_kernel(Mp2Args g) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) evb[e] = (double)g.ev[min(b0 + e, nvir - 1)];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const double ea = eo - (double)g.ev[min(a0 + 16 * u, nvir - 1)];
+    for (int u = 0; u < NU; ++u) {
+      const double ea = eo - (double)g.ev[min(a0 + RS * u, nvir - 1)];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const double tab = x[u][e], tba = y[(c4 + e) * P + r0 + 16 * u];
+        const double tab = x[u][e], tba = y[(c4 + e) * P + r0 + RS * u];
         const double d = ea - evb[e];
         const double w = diag ? tab * fma(2.0, tab, -tba)
                               : 2.0 * fma(tab, tab, tba * (tba - tab));
-        if (a0 + 16 * u < nvir && b0 + e < nvir) sum += w / d;
+        if (a0 + RS * u < nvir && b0 + e < nvir) sum += w / d;
       }
     }
   }
@@ -1882,8 +1890,8 @@ extern "C" int trnblas_hip_mp2_energy_split(int64_t ic, int64_t nocc, int64_t nv
     TRNBLAS_CHECK_ARG(T_flat && eps_vir && ldt >= nocc * nvir, "mp2_energy: bad T_flat / ldt");
   const Mp2Args g{(int)nocc, (int)nvir, (int)nsplit, (int)(ic * nocc), T_flat, ldt,
                   eps_occ_chunk, eps_occ_full, eps_vir, out};
-  hipLaunchKernelGGL(mp2_energy_kernel, dim3((unsigned)(ic * nocc * nsplit)), dim3(256), 0,
-                     (hipStream_t)stream, g);
+  hipLaunchKernelGGL(nvir <= kMp2SmallNvir ? mp2_energy_kernel<32> : mp2_energy_kernel<64>,
+                     dim3((unsigned)(ic * nocc * nsplit)), dim3(256), 0, (hipStream_t)stream, g);
   return check_launch("mp2_energy");
 }
 

@@ -540,7 +540,6 @@ def pair_energies(
 # Workgroups of an mp2_energy launch: eight per CU (four waves each, which
 # hide the loads of each other's tile pairs); blocks of fewer pairs are split.
 _MP2_GROUPS = 2048
-_MP2_TILE = 64
 
 
 def mp2_energy_partials(T_flat, eps_occ_chunk, eps_occ_full, eps_vir) -> torch.Tensor:
@@ -553,7 +552,7 @@ def mp2_energy_partials(T_flat, eps_occ_chunk, eps_occ_full, eps_vir) -> torch.T
     if T_flat.stride(1) != 1:
         T_flat = T_flat.contiguous()
     ic, nocc, nvir = eps_occ_chunk.numel(), eps_occ_full.numel(), eps_vir.numel()
-    nb = -(-nvir // _MP2_TILE)
+    nb = -(-nvir // (32 if nvir <= 256 else 64))  # the kernel's tiles
     nsplit = max(1, min(nb * (nb + 1) // 2, -(-_MP2_GROUPS // max(1, ic * nocc))))
     out = torch.empty((ic * nocc, nsplit), dtype=torch.float64, device=dev)
     f32 = torch.float32
